@@ -276,6 +276,32 @@ def test_grid_sample(gpu, name):
     assert bool((nb3 == -1).all()) and bool((wt3 == 0).all())
 
 
+@pytest.mark.parametrize("L", [1, 31, 32, 33, 63, 65, 4000])
+def test_grid_sample_ragged(gpu, L):
+    """Point counts around the sample map's 64-point workgroup, points that are not finite among them: rows and
+    weights equal those of the same points inside a longer call, nothing is written past L, and the normalized weights
+    are the corner-order sum's quotients. Sums for channel counts of every vector width, reading an x at a 4-byte
+    offset, are the float32 fused multiply-add chain: within 8 roundings of the float64 sum."""
+    c = coords("c1")
+    rng = np.random.default_rng(11)
+    pts = rng.uniform(-1.0, 33.0, size=(4100, 3)).astype(np.float32)
+    pts[5], pts[17, 1], pts[30, 2] = np.nan, np.inf, -3e38
+    tp = torch.from_numpy(pts).to(gpu)
+    cache = sp.build_neighbors(torch.from_numpy(c).to(gpu), 32, 32, 32, keep_hash=True)
+    for norm in (False, True):
+        nb, wt = sp.grid_sample_map(cache, tp, normalize=norm)
+        nbL, wtL = sp.grid_sample_map(cache, tp[:L], normalize=norm)
+        assert torch.equal(nbL, nb[:L]) and torch.equal(wtL, wt[:L])
+        bad = [i for i in (5, 17, 30) if i < L]
+        assert bool((nbL[bad] == -1).all()) and bool((wtL[bad] == 0).all())
+    nb, wt = sp.grid_sample_map(cache, tp[:L])
+    for C in (1, 2, 3, 4, 6, 8, 12):
+        x = torch.from_numpy(rng.standard_normal(len(c) * C + 1).astype(np.float32)).to(gpu)[1:].view(len(c), C)
+        y = sp.grid_sample_sum(x, nb, wt).double()
+        xv = torch.where((nb >= 0)[:, :, None], x[nb.clamp(min=0).long()], 0.0).double() * wt.double()[:, :, None]
+        assert bool(((y - xv.sum(1)).abs() <= 8 * 2.0 ** -24 * xv.abs().sum(1) + 1e-30).all()), C
+
+
 @pytest.mark.parametrize("name", ["c1", "c5"])
 def test_subdivide_build(gpu, name):
     """subdivide_build (no host sync between the subdivision and the map build: launches sized for the 8n-child
