@@ -75,6 +75,23 @@ def test_convnext_mlp_many_tiles_in_place(gpu, C):
     check(hg, (h, x, None, None, w1, None, w2, None), 1e-5, torch.bfloat16, f"C={C} N={N} in place")
 
 
+@pytest.mark.parametrize("C,N", [(256, 1), (256, 127), (256, 129), (256, 5003), (256, 33000), (512, 128), (512, 2600),
+                                 (1024, 65), (1024, 1217), (1024, 2049), (1024, 24700)])
+def test_convnext_mlp_wide_tiles(gpu, C, N):
+    """The LayerNorm + two-GEMM form around its 64- and 128-row tiles and in each of its tile shapes (by rows and K:
+    64 x 128 with two K groups, 128 x 128, 128 x 256), and with the rows in two parts (N = 24700 at C = 1024); no
+    row past N is written. Same bounds as above, against torch fp32 on the GPU."""
+    args = make(N, C, torch.float16, torch.float32, C + N)
+    dev = [a.to(gpu) for a in args]
+    out = torch.full((N + 3, C), 7.0, dtype=torch.float16, device=gpu)
+    y = sp.convnext_mlp(*dev, eps=1e-6, out=out[:N])
+    em, f32 = reference(*dev, 1e-6, torch.float16), reference(*dev, 1e-6)
+    r_em, mx, r_32 = rel(y.float(), em), float((y.float() - em).abs().max()), rel(y.float(), f32)
+    print(f"C={C} N={N}: rel-L2 {r_em:.2e} max-abs {mx:.2e} vs emulated, rel-L2 {r_32:.2e} vs fp32", flush=True)
+    assert r_em <= 2e-3 and mx <= 3e-2 and r_32 <= 1e-2
+    assert bool((out[N:] == 7.0).all())
+
+
 def test_convnext_mlp_errors(gpu):
     h = torch.zeros((10, 96), dtype=torch.bfloat16, device=gpu)
     w1 = torch.zeros((384, 96), dtype=torch.bfloat16, device=gpu)
