@@ -419,12 +419,13 @@ __device__ __forceinline__ void store_row8(const Epi& e, uint32_t o, bool ok, fl
 // Epilogue of one 32-row x 64-channel accumulator group, staged through LDS so every lane writes 16 contiguous
 // bytes: out[order[r], co] = act(acc + b) [+ residual]. `ew` is this wavefront's private [32][72] fp32 area.
 // Residual loads of one 32-row group (4 rows per lane slot p): RK 0 none, 1 fp32, 2 bf16/f16.
-template <int RK, bool NEG = false>
+// (TN = 2: 64 channels, 8 rows per slot p; TN = 1: 32 channels, 16 rows per slot, two slots)
+template <int RK, bool NEG = false, int TN = 2>
 __device__ __forceinline__ void load_group_res(const Epi& e, const int* tile_order, int rbase, int nrows, int Co,
                                                int col, int lane, u32x4 (&r)[4][2]) {
 #pragma unroll
-  for (int p = 0; p < 4; p++) {
-    const int rr = rbase + p * 8 + (lane >> 3);
+  for (int p = 0; p < 2 * TN; p++) {
+    const int rr = rbase + p * (16 / TN) + lane / (4 * TN);
     const uint32_t o = (uint32_t)tile_order[rr] * (uint32_t)Co + (uint32_t)col;
     const bool ok = rr < nrows && (!NEG || tile_order[rr] >= 0);
     r[p][0] = r[p][1] = u32x4{0, 0, 0, 0};
@@ -443,9 +444,10 @@ template <int TN, int TA = TN, int T0 = 0, bool NEG = false>
 __device__ __forceinline__ void epilogue_group(const f32x16 (&acc)[TA], float* ew, const int* tile_order, int rbase,
                                                int nrows, int col, const float (&bias8)[8], const Epi& e, int Co,
                                                int lane, const u32x4 (&r)[4][2]) {
-  constexpr int ES = 72;  // row stride in floats: 4 rows apart differ by 32 banks, so the scatter is conflict-free
+  constexpr int ES = TN * 32 + 8;  // row stride in floats: 4 rows apart differ by 32 banks, so the scatter is
+                                   // conflict-free
   const int h = lane >> 5, l32 = lane & 31;
-  const int c8 = (lane & 7) * 8;
+  const int c8 = lane % (4 * TN) * 8;
 #pragma unroll
   for (int t = 0; t < TN; t++)
 #pragma unroll
@@ -453,8 +455,8 @@ __device__ __forceinline__ void epilogue_group(const f32x16 (&acc)[TA], float* e
   __builtin_amdgcn_wave_barrier();
   asm volatile("" ::: "memory");
 #pragma unroll
-  for (int p = 0; p < 4; p++) {
-    const int rr = p * 8 + (lane >> 3);
+  for (int p = 0; p < 2 * TN; p++) {
+    const int rr = p * (16 / TN) + lane / (4 * TN);
     float v[8];
     *(f32x4*)&v[0] = *(const f32x4*)&ew[rr * ES + c8];
     *(f32x4*)&v[4] = *(const f32x4*)&ew[rr * ES + c8 + 4];
@@ -475,223 +477,20 @@ template <int TM, int TN, int TA = TN, int T0 = 0, bool NEG = false>
 __device__ __forceinline__ void epilogue_tile(const f32x16 (&acc)[TM][TA], float* ew, const int* tile_order,
                                               int nrows, int co_w, const float (&bias8)[8], const Epi& e, int Co,
                                               int lane) {
-  const int col = co_w + (lane & 7) * 8;
+  const int col = co_w + lane % (4 * TN) * 8;
   auto run = [&](auto RKc) __attribute__((always_inline)) {
     constexpr int RK = decltype(RKc)::value;
     u32x4 r[2][4][2];
-    load_group_res<RK, NEG>(e, tile_order, 0, nrows, Co, col, lane, r[0]);
+    load_group_res<RK, NEG, TN>(e, tile_order, 0, nrows, Co, col, lane, r[0]);
     static_for<TM>([&](auto I) __attribute__((always_inline)) {
       if constexpr (I + 1 < TM)
-        load_group_res<RK, NEG>(e, tile_order, (I + 1) * 32, nrows, Co, col, lane, r[(I + 1) & 1]);
+        load_group_res<RK, NEG, TN>(e, tile_order, (I + 1) * 32, nrows, Co, col, lane, r[(I + 1) & 1]);
       epilogue_group<TN, TA, T0, NEG>(acc[I], ew, tile_order, I * 32, nrows, col, bias8, e, Co, lane, r[I & 1]);
     });
   };
   if (e.res_dt < 0) run(std::integral_constant<int, 0>{});
   else if (e.res_dt == F32) run(std::integral_constant<int, 1>{});
   else run(std::integral_constant<int, 2>{});
-}
-
-// Wide-channel kernel: BM sorted rows x BN = 64*NW channels, NW wavefronts; each wavefront owns all BM rows x its
-// own 64 channels (BM/32 x 2 tiles of 32x32 fp32 accumulators).
-//  * Traffic: per K stage (one offset v x 64 input channels) a workgroup reads BM gathered rows and BN weight rows
-//    of 128 bytes, for 2*BM*BN*64 flops; BM = BN = 256 keeps this at 0.0078 byte/flop, which L2 can feed.
-//  * Skipping: the K loop runs over the union of the tile's neighbour masks, but each 32-row group has its own
-//    mask and skips its MFMAs for offsets none of its rows has, so padding work follows 32-row granularity.
-//  * Software pipeline: stage s issues the gather loads of A(s+2) and the weight loads of B(s+1), runs the MFMAs of
-//    stage s (A(s) from LDS, B(s) from registers), then writes A(s+1) -- loaded a full stage earlier -- into the
-//    other LDS buffer and synchronises. The loop is unrolled by two so registers and buffers have fixed names.
-//  * Only A is shared by the wavefronts, so only A goes through LDS; weights (L2-resident) stream straight into
-//    MFMA operand registers. At tile start the offset list, the 32-row masks, the tile's output row indices and its
-//    [BM x 27] neighbour indices are staged in LDS: the K loop has no dependent global loads. EMPTY neighbours
-//    read past the end of the feature buffer, so every gather is an unconditional 16-byte load.
-//  * LDS layout of a stage: row r occupies 128 contiguous bytes as eight 16-byte slots; channel piece p of row r is
-//    stored in slot p ^ (r & 7) so the MFMA operand reads (32 rows, one piece) hit distinct banks.
-//  * Within a 64-channel stage the K order is permuted (lane half h, step j -> piece h*4 + j) identically for A and
-//    B, so each lane's four weight loads are one contiguous 64-byte run.
-//  * Epilogue: per 32-row group, accumulators go through LDS and leave as 16-byte row segments (bias, SiLU,
-//    residual fused, one rounding).
-template <bool F16, int NW, int BM>
-__global__ void __launch_bounds__(NW * 64) k_conv_wide(ConvArgs a) {
-  constexpr int NT = NW * 64, KC = 64, PC = KC / 8;
-  constexpr int TM = BM / 32, TN = 2, AL = BM * PC / NT;  // AL gather loads per lane per stage
-  static_assert(AL * NT == BM * PC && TM <= 8, "tile shape");
-  __shared__ __attribute__((aligned(16))) u32x4 As[2][BM * PC];
-  __shared__ uint32_t srcT[BM * 27];
-  __shared__ int ordT[BM];
-  __shared__ uint32_t gmask[TM];
-  __shared__ int vlist[32];
-
-  const int g = blockIdx.x, per = a.grid / 8;
-  const int logical = (g % 8) * per + g / 8;
-  if (logical >= a.tiles_m * a.tiles_n) return;
-  const int tm_ = logical / a.tiles_n, tn_ = logical % a.tiles_n;
-  const int row0 = tm_ * BM, co0 = tn_ * (64 * NW);
-  const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31, wn = tid >> 6;
-  const int N = a.N, Ci = a.Ci, nkc = Ci / KC;
-
-  // prologue: row indices, 32-row masks (OR of the rows' neighbour masks), offset list, neighbour table
-  for (int r = tid; r < BM; r += NT) {
-    const int row = row0 + r;
-    const int o = row < N ? a.order[row] : 0;
-    ordT[r] = o;
-    uint32_t gm = row < N ? (uint32_t)a.gray[o] : 0u;
-#pragma unroll
-    for (int d = 1; d < 32; d <<= 1) gm |= (uint32_t)__shfl_xor((int)gm, d, 64);
-    if ((r & 31) == 0) gmask[r >> 5] = gm;
-  }
-  __syncthreads();
-  uint32_t mask = 0;
-#pragma unroll
-  for (int i = 0; i < TM; i++) mask |= gmask[i];
-  const int nvv = __popc(mask), total = nvv * nkc;
-  if (tid < 27 && ((mask >> tid) & 1u)) vlist[__popc(mask & ((1u << tid) - 1u))] = tid;
-  const uint32_t row_bytes = (uint32_t)Ci * 2u;
-  // one row per thread: its 27 neighbour indices are one contiguous 108-byte run, loaded as 27 independent loads
-  for (int r = tid; r < BM; r += NT) {
-    uint32_t src[27];
-    const bool live = row0 + r < N;
-    const uint32_t* nrow = a.nbr + (i64)ordT[r] * 27;
-#pragma unroll
-    for (int v = 0; v < 27; v++) src[v] = live ? nrow[v] : EMPTY;
-#pragma unroll
-    for (int v = 0; v < 27; v++) srcT[r * 27 + v] = src[v] == EMPTY ? kOutOfRange : src[v] * row_bytes;
-  }
-  uint32_t gms[TM];
-#pragma unroll
-  for (int i = 0; i < TM; i++) gms[i] = __builtin_amdgcn_readfirstlane(gmask[i]);
-  __syncthreads();
-
-  // this lane's gather pieces: LDS unit u = k*NT + tid -> row u/8, slot u%8, channel piece slot ^ (row & 7)
-  int arow[AL], apiece[AL];
-#pragma unroll
-  for (int k = 0; k < AL; k++) {
-    int u = k * NT + tid;
-    arow[k] = u >> 3;
-    apiece[k] = (u & 7) ^ ((arow[k] >> 1) & 7);
-  }
-  // buffer resources: 32-bit offsets, and gathers of EMPTY neighbours (offset kOutOfRange) return zeros
-  const __amdgpu_buffer_rsrc_t rx = make_rsrc(a.x, a.x_bytes), rw = make_rsrc(a.w, a.w_bytes);
-  // packed weights: the stage (v, kc) fragment of this wavefront's 64-channel slice is 8 KiB at
-  // ((slice*27 + v)*nkc + kc) * 8 KiB, as [t][j][lane][16 bytes]
-  const uint32_t wslice = (uint32_t)((co0 >> 6) + wn) * 27u * (uint32_t)nkc;
-  const uint32_t wlane = (uint32_t)lane * 16u;
-
-  // stage cursors (offset index, channel block); loads past the last stage re-read the last stage
-  int avi = 0, akc = 0, bvi = 0, bkc = 0, cvi = 0, ckc = 0;
-  auto next = [&](int& vi, int& kc) __attribute__((always_inline)) {
-    const bool wrap = kc + 1 == nkc;
-    kc = wrap ? 0 : kc + 1;
-    vi += wrap ? 1 : 0;
-  };
-  auto load_a = [&](u32x4 (&ra)[AL]) __attribute__((always_inline)) {
-    const bool live = avi < nvv;
-    const int v = __builtin_amdgcn_readfirstlane(vlist[live ? avi : nvv - 1]);
-    const int k0 = __builtin_amdgcn_readfirstlane((live ? akc : nkc - 1) * KC);
-    uint32_t off[AL];
-#pragma unroll
-    for (int k = 0; k < AL; k++) off[k] = srcT[arow[k] * 27 + v];
-#pragma unroll
-    for (int k = 0; k < AL; k++)
-      ra[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, off[k] + apiece[k] * 16, k0 * 2, 0);
-    next(avi, akc);
-  };
-  auto store_a = [&](int buf, const u32x4 (&ra)[AL]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int k = 0; k < AL; k++) As[buf][k * NT + tid] = ra[k];
-  };
-  auto load_b = [&](u32x4 (&rb)[TN][4]) __attribute__((always_inline)) {
-    const bool live = bvi < nvv;
-    const int v = __builtin_amdgcn_readfirstlane(vlist[live ? bvi : nvv - 1]);
-    const int k0 = __builtin_amdgcn_readfirstlane((live ? bkc : nkc - 1) * KC);
-    const int soff = __builtin_amdgcn_readfirstlane((int)((wslice + (uint32_t)(v * nkc) + (uint32_t)(k0 / KC)) * 8192u));
-#pragma unroll
-    for (int t = 0; t < TN; t++)
-#pragma unroll
-      for (int j = 0; j < 4; j++) rb[t][j] = __builtin_amdgcn_raw_buffer_load_b128(rw, wlane + (t * 4 + j) * 1024, soff, 0);
-    next(bvi, bkc);
-  };
-
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int i = 0; i < TM; i++)
-#pragma unroll
-    for (int t = 0; t < TN; t++) acc[i][t] = f32x16{};
-  // One K stage, with the next stages' traffic interleaved between the MFMA groups so the vector-memory and LDS
-  // queues drain while the matrix cores run: group i issues its share of the A(s+2) gathers and B(s+1) weight
-  // loads, writes its share of A(s+1) (loaded a stage ago) into the other LDS buffer, prefetches the operands of
-  // group i+1, then runs its MFMAs if any of its 32 rows has offset v.
-  auto stage = [&](int buf, const u32x4 (&rbC)[TN][4], const u32x4 (&raW)[AL], u32x4 (&raL)[AL],
-                   u32x4 (&rbN)[TN][4]) __attribute__((always_inline)) {
-    const uint32_t vbit = 1u << __builtin_amdgcn_readfirstlane(vlist[cvi]);
-    next(cvi, ckc);
-    // A(s+2) addresses
-    const bool alive = avi < nvv;
-    const int va = __builtin_amdgcn_readfirstlane(vlist[alive ? avi : nvv - 1]);
-    const int ka = __builtin_amdgcn_readfirstlane((alive ? akc : nkc - 1) * KC * 2);
-    next(avi, akc);
-    uint32_t off[AL];
-#pragma unroll
-    for (int k = 0; k < AL; k++) off[k] = srcT[arow[k] * 27 + va] + apiece[k] * 16;
-    // B(s+1) base
-    const bool blive = bvi < nvv;
-    const int vb = __builtin_amdgcn_readfirstlane(vlist[blive ? bvi : nvv - 1]);
-    const int kb = blive ? bkc : nkc - 1;
-    const int soff = __builtin_amdgcn_readfirstlane((int)((wslice + (uint32_t)(vb * nkc + kb)) * 8192u));
-    next(bvi, bkc);
-
-    u32x4 fa[2][4];
-    auto read_fa = [&](u32x4 (&f)[4], int i) __attribute__((always_inline)) {
-      const int r = i * 32 + l32;
-#pragma unroll
-      for (int j = 0; j < 4; j++) f[j] = As[buf][r * PC + ((h * 4 + j) ^ ((r >> 1) & 7))];
-    };
-    read_fa(fa[0], 0);
-    constexpr int AG = AL / TM, BG = TN * 4 / TM;  // loads per group
-    static_assert(AG * TM == AL && BG * TM == TN * 4 && BG >= 1, "load split");
-#pragma unroll
-    for (int i = 0; i < TM; i++) {
-#pragma unroll
-      for (int k = i * AG; k < (i + 1) * AG; k++) raL[k] = __builtin_amdgcn_raw_buffer_load_b128(rx, off[k], ka, 0);
-#pragma unroll
-      for (int q = i * BG; q < (i + 1) * BG; q++)
-        rbN[q / 4][q % 4] = __builtin_amdgcn_raw_buffer_load_b128(rw, wlane + q * 1024, soff, 0);
-#pragma unroll
-      for (int k = i * AG; k < (i + 1) * AG; k++) As[buf ^ 1][k * NT + tid] = raW[k];
-      if (i + 1 < TM) read_fa(fa[(i + 1) & 1], i + 1);
-      if (gms[i] & vbit) {
-#pragma unroll
-        for (int j = 0; j < 4; j++)
-#pragma unroll
-          for (int t = 0; t < TN; t++) acc[i][t] = mfma32<F16>(fa[i & 1][j], rbC[t][j], acc[i][t]);
-      }
-    }
-    __syncthreads();
-  };
-
-  if (total > 0) {
-    u32x4 ra0[AL], ra1[AL], rb0[TN][4], rb1[TN][4];
-    load_a(ra0);  // A(0)
-    load_b(rb0);  // B(0)
-    load_a(ra1);  // A(1)
-    store_a(0, ra0);
-    __syncthreads();
-    for (int s = 0; s < total; s += 2) {
-      stage(0, rb0, ra1, ra0, rb1);  // MFMAs of stage s; writes A(s+1); loads A(s+2), B(s+1)
-      if (s + 1 >= total) break;
-      stage(1, rb1, ra0, ra1, rb0);  // stage s+1; writes A(s+2); loads A(s+3), B(s+2)
-    }
-  }
-
-  // epilogue through this wavefront's share of the (now idle) A buffers
-  float* ew = (float*)&As[0][0] + wn * (32 * 72);
-  static_assert(NW * 32 * 72 * 4 <= 2 * BM * PC * 16, "epilogue staging fits in the A buffers");
-  const int co_w = co0 + wn * 64;
-  float bias8[8];
-#pragma unroll
-  for (int q = 0; q < 8; q++) bias8[q] = a.bias ? a.bias[co_w + (lane & 7) * 8 + q] : 0.f;
-  const int nrows = N - row0;
-  const Epi e = make_epi(a);
-  epilogue_tile<TM, TN>(acc, ew, ordT, nrows, co_w, bias8, e, a.Co, lane);
 }
 
 typedef float f32x4v __attribute__((ext_vector_type(4)));
@@ -1376,25 +1175,39 @@ void launch_narrow(ConvArgs a, hipStream_t st = stream()) {
   else k_conv_narrow<F16, S, T, G><<<a.grid, 256, 0, st>>>(a);
 }
 
-// Wide-channel kernel, BM sorted rows x 256 channels per workgroup (4 wavefronts, each all BM rows x 64 channels =
-// BM/32 x 2 tiles of 32x32 fp32 accumulators). BM = 128 is the one launched: two workgroups per CU, so one
-// workgroup's prologue, barriers and epilogue overlap the other's MFMAs. Differences from k_conv_wide:
+// Wide-channel kernel: 128 sorted rows x 128 TN channels per workgroup (TN = 2, or 1 where Co is an odd multiple of
+// 128), 4 wavefronts, each all 128 rows x its own 32 TN channels (4 x TN tiles of 32x32 fp32 accumulators), 4 - TN
+// workgroups per CU, so one workgroup's prologue, barriers and epilogue overlap the others' MFMAs. TN = 1 reads each
+// gathered byte from LDS for half the flops and waits more, so a third workgroup per CU (a ring of two slots) pays
+// more there than gathers three stages ahead: 391007 rows of 128 -> 128, 285 us against ~300 with four slots and two
+// workgroups, and 385 for the former kernel of 128 rows x 128 channels staged through registers.
+//  * Skipping: the K loop runs over the union of the tile's neighbour masks, but each 32-row group has its own mask and
+//    skips its MFMAs for offsets none of its rows has, so padding work follows 32-row granularity.
+//  * Only A is shared by the wavefronts, so only A goes through LDS; weights (L2-resident) stream straight into MFMA
+//    operand registers. At tile start the offset list, the 32-row masks, the tile's output row indices and its
+//    [128 x 27] neighbour indices are staged in LDS: the K loop has no dependent global loads.
+//  * LDS layout of a stage: row r occupies 128 contiguous bytes as eight 16-byte slots; channel piece p of row r is in
+//    slot p ^ ((r >> 1) & 7), so the MFMA operand reads (32 rows, one piece) hit distinct banks. Within a 64-channel
+//    stage the K order is permuted (lane half h, step j -> piece h*4 + j) identically for A and B.
+//  * Epilogue: per 32-row group, accumulators go through LDS and leave as 16-byte row segments.
 //  * The gathered A tile goes global -> LDS directly (buffer_load ... lds, 16 bytes per lane; EMPTY neighbours
-//    read past the buffer end and land as zeros) into a 4-slot LDS ring, 3 stages ahead of the MFMAs: no
-//    registers hold gathers in flight, and gather latency hides behind three stages of MFMA work. The slots are
-//    four distinct LDS objects so the compiler can tell the DMA into one slot from the reads of another.
+//    read past the buffer end and land as zeros) into an LDS ring of NS slots (4, or 2 at TN = 1), NS - 1
+//    stages ahead of the MFMAs: no registers hold gathers in flight. The slots are
+//    distinct LDS objects so the compiler can tell the DMA into one slot from the reads of another.
 //  * Ring protocol per stage s: wait (counted vmcnt) for this lane's DMA of A(s), barrier (every wavefront's
-//    part has landed and everyone is done with stage s-1), then refill the slot stage s-1 used with A(s+3).
+//    part has landed and everyone is done with stage s-1), then refill the slot stage s-1 used with A(s+NS-1).
 //  * K-step-outer MFMA order: for each 16-wide K step j of the stage, the MFMAs of every 32-row group, then the
 //    weights of stage s+1 for step j go into the registers step j just released. One weight register set (not two),
 //    a stage of latency slack for every weight load, and BM/32 x 2 independent accumulator chains in flight.
-template <bool F16, int BM>
-__global__ void __launch_bounds__(256, BM == 128 ? 2 : 1) k_conv_wide_dma(ConvArgs a) {
+template <bool F16, int BM, int TN>
+__global__ void __launch_bounds__(256, 4 - TN) k_conv_wide_dma(ConvArgs a) {
   constexpr int NW = 4, NT = 256, KC = 64, PC = KC / 8;
-  constexpr int TM = BM / 32, TN = 2, AL = BM * PC / NT;  // TM groups of 32 rows per wavefront
+  constexpr int TM = BM / 32, AL = BM * PC / NT;  // TM groups of 32 rows per wavefront, TN of 32 channels
+  constexpr int NBL = 4 * TN, NS = TN == 1 ? 2 : 4;  // weight loads per stage, ring slots
   static_assert(AL == TM, "one A DMA per 32-row group");
-  static_assert(BM == 128 || BM == 256, "tile rows");
-  __shared__ __attribute__((aligned(16))) u32x4 As0[BM * PC], As1[BM * PC], As2[BM * PC], As3[BM * PC];
+  static_assert(BM == 128 && (TN == 1 || TN == 2), "tile");
+  __shared__ __attribute__((aligned(16))) u32x4 As0[BM * PC], As1[BM * PC], As2[NS == 4 ? BM * PC : 1],
+      As3[NS == 4 ? BM * PC : 1];
   __shared__ uint32_t srcT[BM * 27];
   __shared__ int ordT[BM];
   __shared__ uint32_t gmask[BM / 32];
@@ -1429,7 +1242,7 @@ __global__ void __launch_bounds__(256, BM == 128 ? 2 : 1) k_conv_wide_dma(ConvAr
   const bool tmaj = a.tnmaj;  // set only with the tail-split schedule (no tsched)
   const int tm_ = a.tsched && !a.part ? a.tsched[logical / a.tiles_n] : tmaj ? logical % a.tiles_m : logical / a.tiles_n;
   const int tn_ = tmaj ? logical / a.tiles_m : logical % a.tiles_n;
-  const int row0 = tm_ * BM, co0 = tn_ * (64 * NW);
+  const int row0 = tm_ * BM, co0 = tn_ * (32 * TN * NW);
   const int tid = threadIdx.x, lane = tid & 63, h = lane >> 5, l32 = lane & 31;
   const int wv = __builtin_amdgcn_readfirstlane(tid >> 6), wn = wv;
   const int N = a.N, Ci = a.Ci, nkc = Ci / KC;
@@ -1469,8 +1282,9 @@ __global__ void __launch_bounds__(256, BM == 128 ? 2 : 1) k_conv_wide_dma(ConvAr
     drow[k] = u >> 3;
     dpiece[k] = (u & 7) ^ ((u >> 4) & 7);
   }
-  const uint32_t wslice = (uint32_t)((co0 >> 6) + wn) * 27u * (uint32_t)nkc;
-  const uint32_t wlane = (uint32_t)lane * 16u;
+  const int co_w = co0 + wn * (32 * TN);  // this wavefront's first channel, and its place in the 64-channel blocks
+  const uint32_t wslice = (uint32_t)(co_w >> 6) * 27u * (uint32_t)nkc;
+  const uint32_t wlane = (uint32_t)lane * 16u + (uint32_t)(co_w & 32) * 128u;
 
   // K stages run channel block outer, offset inner: stage s = (kc = s / nvv, offset entry vi = s % nvv). A row chunk
   // gathered for one offset is then gathered again for the next offset's (one voxel over) neighbours one stage
@@ -1509,7 +1323,7 @@ __global__ void __launch_bounds__(256, BM == 128 ? 2 : 1) k_conv_wide_dma(ConvAr
 #pragma unroll
     for (int t = 0; t < TN; t++) acc[i][t] = f32x16{};
 
-  // one K stage: MFMAs from slot `cur` and the weights in rb (stage s); DMA A(s+3) into `fill`; rb refilled with
+  // one K stage: MFMAs from slot `cur` and the weights in rb (stage s); DMA A(s+NS-1) into `fill`; rb refilled with
   // the weights of stage s+1, K step by K step
   auto stage = [&](const u32x4* cur, u32x4* fill, u32x4 (&rb)[TN][4]) __attribute__((always_inline)) {
     const uint32_t vbit = 1u << __builtin_amdgcn_readfirstlane(vlist[cvi]);
@@ -1548,14 +1362,14 @@ __global__ void __launch_bounds__(256, BM == 128 ? 2 : 1) k_conv_wide_dma(ConvAr
         rb[t][j] = __builtin_amdgcn_raw_buffer_load_b128(rw, wlane + (t * 4 + j) * 1024, soff, 0);
     }
   };
-  // loads issued after this lane's last DMA of A(s) when stage s starts: prologue DMAs and B(0) for s < 3,
-  // then (in steady state) the last K step's TN weight loads of stage s-3 plus two full stages of AL + 8
-  constexpr int SL = AL + 8;
+  // loads issued after this lane's last DMA of A(s) when stage s starts: prologue DMAs and B(0) for s < NS - 1,
+  // then (in steady state) the last K step's TN weight loads of stage s-NS+1 plus NS - 2 full stages of AL + NBL
+  constexpr int SL = AL + NBL;
   auto wait_a = [&](int s) __attribute__((always_inline)) {
-    if (s == 0) wait_vmcnt<2 * AL + 8>();
-    else if (s == 1) wait_vmcnt<AL + 8 + SL>();
-    else if (s == 2) wait_vmcnt<8 + 2 * SL>();
-    else wait_vmcnt<TN + 2 * SL>();
+    if (s == 0) wait_vmcnt<(NS - 2) * AL + NBL>();
+    else if (NS == 4 && s == 1) wait_vmcnt<AL + NBL + SL>();
+    else if (NS == 4 && s == 2) wait_vmcnt<NBL + 2 * SL>();
+    else wait_vmcnt<TN + (NS - 2) * SL>();
   };
 
   if (total > 0) {
@@ -1566,55 +1380,59 @@ __global__ void __launch_bounds__(256, BM == 128 ? 2 : 1) k_conv_wide_dma(ConvAr
       a_offsets(off, ka);
 #pragma unroll
       for (int k = 0; k < AL; k++) dma(As0, k, off[k], ka);
-      a_offsets(off, ka);
+      if constexpr (NS == 4) {
+        a_offsets(off, ka);
 #pragma unroll
-      for (int k = 0; k < AL; k++) dma(As1, k, off[k], ka);
-      a_offsets(off, ka);
+        for (int k = 0; k < AL; k++) dma(As1, k, off[k], ka);
+        a_offsets(off, ka);
 #pragma unroll
-      for (int k = 0; k < AL; k++) dma(As2, k, off[k], ka);
+        for (int k = 0; k < AL; k++) dma(As2, k, off[k], ka);
+      }
       const int soff = b_base();
 #pragma unroll
-      for (int q = 0; q < 8; q++) rb[q / 4][q % 4] = __builtin_amdgcn_raw_buffer_load_b128(rw, wlane + q * 1024, soff, 0);
+      for (int q = 0; q < NBL; q++) rb[q / 4][q % 4] = __builtin_amdgcn_raw_buffer_load_b128(rw, wlane + q * 1024, soff, 0);
     }
-    for (int s = 0; s < total; s += 4) {
+    for (int s = 0; s < total; s += NS) {
       wait_a(s);
       wg_barrier();
-      stage(As0, As3, rb);
+      stage(As0, NS == 4 ? As3 : As1, rb);
       if (s + 1 >= total) break;
       wait_a(s + 1);
       wg_barrier();
       stage(As1, As0, rb);
-      if (s + 2 >= total) break;
-      wait_a(s + 2);
-      wg_barrier();
-      stage(As2, As1, rb);
-      if (s + 3 >= total) break;
-      wait_a(s + 3);
-      wg_barrier();
-      stage(As3, As2, rb);
+      if constexpr (NS == 4) {
+        if (s + 2 >= total) break;
+        wait_a(s + 2);
+        wg_barrier();
+        stage(As2, As1, rb);
+        if (s + 3 >= total) break;
+        wait_a(s + 3);
+        wg_barrier();
+        stage(As3, As2, rb);
+      }
     }
   }
   wait_vmcnt<0>();
   if (pslot >= 0) {  // a piece of a split tile: its fp32 partial sums go to the workspace, the reduction does the rest
-    float* pp = a.part + (size_t)pslot * (BM * 256);
+    float* pp = a.part + (size_t)pslot * (BM * 128 * TN);
 #pragma unroll
     for (int i = 0; i < TM; i++)
 #pragma unroll
       for (int t = 0; t < TN; t++)
 #pragma unroll
         for (int q = 0; q < 16; q++)
-          pp[(i * 32 + (q >> 2) * 8 + h * 4 + (q & 3)) * 256 + wn * 64 + t * 32 + l32] = acc[i][t][q];
+          pp[(i * 32 + (q >> 2) * 8 + h * 4 + (q & 3)) * (128 * TN) + wn * (32 * TN) + t * 32 + l32] = acc[i][t][q];
     return;
   }
   __syncthreads();
 
-  // epilogue through the (now idle) ring: one slot per wavefront
-  float* ew = (float*)(wv == 0 ? &As0[0] : wv == 1 ? &As1[0] : wv == 2 ? &As2[0] : &As3[0]);
+  // epilogue through the (now idle) ring: one slot per wavefront, or half of one
+  float* ew = NS == 4 ? (float*)(wv == 0 ? &As0[0] : wv == 1 ? &As1[0] : wv == 2 ? &As2[0] : &As3[0])
+                      : (float*)(wv < 2 ? &As0[0] : &As1[0]) + (wv & 1) * (32 * 40);
   static_assert(32 * 72 * 4 <= BM * PC * 16, "a wavefront's epilogue staging fits in a ring slot");
-  const int co_w = co0 + wn * 64;
   float bias8[8];
 #pragma unroll
-  for (int q = 0; q < 8; q++) bias8[q] = a.bias ? a.bias[co_w + (lane & 7) * 8 + q] : 0.f;
+  for (int q = 0; q < 8; q++) bias8[q] = a.bias ? a.bias[co_w + lane % (4 * TN) * 8 + q] : 0.f;
   const int nrows = N - row0;
   const Epi e = make_epi(a);
   epilogue_tile<TM, TN>(acc, ew, ordT, nrows, co_w, bias8, e, a.Co, lane);
@@ -2136,11 +1954,11 @@ __global__ void __launch_bounds__(256) k_split_reduce256(ConvArgs a) {
 // for it), as were 8 wavefronts of 128 rows x 64 channels on a 256-row tile (3% slower: weights loaded twice).
 // Reduction of the split tiles: one thread per (row, 8 channels) of a split tile; sums its pieces' partials in
 // piece order, then the fused epilogue (bias, act, residual, one rounding) of the unsplit kernel.
-template <int BM>
+template <int BM, int BN>
 __global__ void __launch_bounds__(256) k_split_reduce(ConvArgs a) {
-  constexpr int UPT = BM * 256 / 8 / 256;  // workgroups per split tile
+  constexpr int UPT = BM * BN / 8 / 256;  // workgroups per split tile
   int st = blockIdx.x / UPT;                 // split tile, counted over the XCDs in order
-  const int e8 = (blockIdx.x % UPT) * 256 + threadIdx.x, r = e8 / 32, c8 = (e8 % 32) * 8;
+  const int e8 = (blockIdx.x % UPT) * 256 + threadIdx.x, r = e8 / (BN / 8), c8 = e8 % (BN / 8) * 8;
   int x = 0, ntail = 0;
   for (; x < 8; x++) {
     ntail = a.xk[x] > 1 ? (a.xt0[x + 1] - a.xt0[x]) - a.xs : 0;
@@ -2151,10 +1969,10 @@ __global__ void __launch_bounds__(256) k_split_reduce(ConvArgs a) {
   const int kx = a.xk[x], logical = a.xt0[x] + a.xs + st, pbase = a.xpart0[x] + st * kx;
   const int tm_ = a.tnmaj ? logical % a.tiles_m : logical / a.tiles_n;
   const int tn_ = a.tnmaj ? logical / a.tiles_m : logical % a.tiles_n;
-  const int row = tm_ * BM + r, col = tn_ * 256 + c8;
+  const int row = tm_ * BM + r, col = tn_ * BN + c8;
   float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
   for (int j = 0; j < kx; j++) {
-    const float* pp = a.part + ((size_t)(pbase + j) * BM + r) * 256 + c8;
+    const float* pp = a.part + ((size_t)(pbase + j) * BM + r) * BN + c8;
     const f32x4 lo = *(const f32x4*)pp, hi = *(const f32x4*)(pp + 4);
 #pragma unroll
     for (int q = 0; q < 4; q++) {
@@ -2193,15 +2011,15 @@ bool split_enabled() {
 // per XCD), the last ones would run as a thin second round; instead each of them is split over k = 64 / tail
 // (at most 8) workgroups along its K stages, so the second round is as wide as the first and k times shorter.
 // Measured on C2: 0.81 ms with 198 row tiles against 0.59 ms with 170 (510 workgroups, one round).
-template <bool F16>
+template <bool F16, int TN>
 void launch_wide_dma(ConvArgs a) {
-  constexpr int BM = 128;
+  constexpr int BM = 128, BN = 128 * TN;
   a.tiles_m = cdiv(a.N, BM);
-  a.tiles_n = a.Co / 256;
+  a.tiles_n = a.Co / BN;
   const int tiles = a.tiles_m * a.tiles_n;
   a.grid = (tiles + 7) / 8 * 8;
   a.part = nullptr;
-  const int slots = 2 * (device_cus() / 8);  // concurrent workgroups per XCD
+  const int slots = (4 - TN) * (device_cus() / 8);  // concurrent workgroups per XCD
   const int per = cdiv(tiles, 8);
   Tensor ws;
   if (split_enabled() && slots > 0 && per > slots && per - slots <= slots / 2) {
@@ -2217,7 +2035,7 @@ void launch_wide_dma(ConvArgs a) {
     }
     a.xt0[8] = tiles;
     if (pslots > 0) {
-      ws = empty({(i64)pslots * BM * 256}, F32);
+      ws = empty({(i64)pslots * BM * BN}, F32);
       a.part = ws.ptr<float>();
       a.grid = 8 * units;
     }
@@ -2236,7 +2054,7 @@ void launch_wide_dma(ConvArgs a) {
     }
     a.xt0[8] = tiles;
     if (pslots > 0) {
-      ws = empty({(i64)pslots * BM * 256}, F32);
+      ws = empty({(i64)pslots * BM * BN}, F32);
       a.part = ws.ptr<float>();
       a.grid = 8 * units;
     }
@@ -2248,12 +2066,12 @@ void launch_wide_dma(ConvArgs a) {
   // 0.800 -> 0.788 ms (three interleaved runs on two boxes; runs of 4 / 8 / 12 / 24 / 32 / 64 / 128 tiles measured
   // 0.795 / 0.793 / 0.792 / 0.793 / 0.792 / 0.798 / 0.815).
   a.xblk = 16;
-  k_conv_wide_dma<F16, BM><<<a.grid, 256, 0, stream()>>>(a);
+  k_conv_wide_dma<F16, BM, TN><<<a.grid, 256, 0, stream()>>>(a);
   if (a.part) {
     int ntail = 0;
     for (int x = 0; x < 8; x++)
       if (a.xk[x] > 1) ntail += (a.xt0[x + 1] - a.xt0[x]) - a.xs;
-    k_split_reduce<BM><<<ntail * (BM * 256 / 8 / 256), 256, 0, stream()>>>(a);
+    k_split_reduce<BM, BN><<<ntail * (BM * BN / 8 / 256), 256, 0, stream()>>>(a);
   }
 }
 
@@ -2317,15 +2135,6 @@ void launch_w256(ConvArgs a) {
   if (ns > 1) k_split_reduce256<<<tiles * 32, 256, 0, stream()>>>(a);
 }
 
-template <bool F16, int NW, int BM>
-void launch_wide(ConvArgs a) {
-  a.tiles_m = cdiv(a.N, BM);
-  a.tiles_n = a.Co / (64 * NW);
-  int tiles = a.tiles_m * a.tiles_n;
-  a.grid = (tiles + 7) / 8 * 8;
-  k_conv_wide<F16, NW, BM><<<a.grid, NW * 64, 0, stream()>>>(a);
-}
-
 // Weight repack for the wide kernel: w [Co,27,Ci] -> one 1 KiB block per (64-channel output slice, offset v,
 // 64-channel input block kc, 32-column half t, step j), laid out as 64 lanes x 16 bytes in MFMA operand order:
 // lane l holds column c = slice*64 + t*32 + (l & 31), input channels kc*64 + (l >> 5)*32 + j*8 .. +8.
@@ -2374,8 +2183,8 @@ void dispatch(const SpConvCfg& cfg, ConvArgs a) {
   }
   // Fixed tiles per channel width (no autotune): BM = 128 sorted rows per tile.
   if (a.Co % 256 == 0 && a.Ci % 64 == 0 && w256_enabled()) return launch_w256<F16>(a);
-  if (cfg.BK == 64 && a.Co % 256 == 0) return launch_wide_dma<F16>(a);
-  if (cfg.BK == 64 && a.Co % 128 == 0) return launch_wide<F16, 2, 128>(a);
+  if (cfg.BK == 64 && a.Co % 256 == 0) return launch_wide_dma<F16, 2>(a);
+  if (cfg.BK == 64 && a.Co % 128 == 0) return launch_wide_dma<F16, 1>(a);
   if (a.Co % 128 == 0) {
     if (cfg.BK == 64) launch<F16, 128, 128, 2, 2, 64>(a);
     else launch<F16, 128, 128, 2, 2, 32>(a);
@@ -2396,7 +2205,7 @@ SpConvCfg spconv_cfg(int N, int Ci, int Co) {
 // them through a row map instead; the others get the gathered rows materialized.
 bool reads_row_table(const SpConvCfg& cfg, int Ci, int Co, int act) {
   (void)act;
-  return (Co == 64 && Ci <= 128) || (cfg.BK == 64 && Co % 256 == 0);
+  return (Co == 64 && Ci <= 128) || (cfg.BK == 64 && Co % 128 == 0);
 }
 
 __global__ void k_gather_rows(const u32x4* __restrict__ x, i64 m, int units, const int32_t* __restrict__ row_map,
@@ -2617,14 +2426,13 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     wpack = empty({(i64)Co * 27 * Ci}, x.dt);
     k_pack_w<<<dim3(Ci / 64 * 2, 27, Co / 64), 256, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci);
     a.w = wpack.ptr<uint16_t>();
-    if (Co % 256 == 0) {  // the 128 x 256 kernel reads its tiles' neighbour rows from the sorted-order table
-      const SpConvCache::RowTable& rt = c.row_table(-1);
-      if (row_map) mtbl = c.mapped_table(-1, *row_map, shift, M);
-      a.tbl = row_map ? mtbl.ptr<uint32_t>() : rt.tbl.ptr<uint32_t>();
-      a.gs = rt.gs.ptr<int32_t>();
-      a.tbl_bytes = (uint32_t)rt.tbl.bytes();
-      a.tsched = c.tile_schedule(-1, 128).ptr<int32_t>();
-    }
+    // the kernel reads its tiles' neighbour rows from the sorted-order table
+    const SpConvCache::RowTable& rt = c.row_table(-1);
+    if (row_map) mtbl = c.mapped_table(-1, *row_map, shift, M);
+    a.tbl = row_map ? mtbl.ptr<uint32_t>() : rt.tbl.ptr<uint32_t>();
+    a.gs = rt.gs.ptr<int32_t>();
+    a.tbl_bytes = (uint32_t)rt.tbl.bytes();
+    a.tsched = c.tile_schedule(-1, 128).ptr<int32_t>();
   }
   REQ(!skip || ht, "the fused skip residual needs the halo kernel");
   REQ(!ln || (ht && ht->host_spills() == 0), "the fused pre-activation needs the halo kernel with no spill tiles");
