@@ -118,6 +118,23 @@ def test_kmap_sort_unpublished_digit_sums(gpu, monkeypatch, limit):
     check_map(c, gpu, B1s=(128,))
 
 
+@pytest.mark.parametrize("n", [1, 63, 1023, 1025, 24576, 24577, 40000])
+def test_sort_small(gpu, n):
+    """Row counts around the sort's 1024-key workgroups and its two forms (one launch per pass up to 24576 keys, three
+    above), rows shuffled: map, masks and order bit-exact; and a subdivision whose children's capacity is n rounded
+    down to 8, equal to subdivide + build_neighbors."""
+    c = coords("c3")[:n].copy()
+    c = c[np.random.default_rng(n).permutation(len(c))]
+    check_map(c, gpu, B1s=(128,))
+    par = torch.from_numpy(c[:max(n // 8, 1)]).to(gpu)
+    lg = torch.from_numpy(W.keep_logits(len(par), 0.4, n).view(np.int16)).to(gpu).view(torch.float16)
+    cc, src, cache = sp.subdivide_build(par, lg)
+    oc, osrc = sp.subdivide(par, lg)
+    assert torch.equal(cc, oc) and torch.equal(src, osrc)
+    for a, b in zip(cache.tensors(), sp.build_neighbors(oc).tensors()):
+        assert torch.equal(a, b)
+
+
 @pytest.mark.parametrize("name", ["c1", "c5"])
 def test_subdivide(gpu, name):
     par = coords(name)

@@ -177,7 +177,7 @@ __global__ void __launch_bounds__(NVV) k_neighbors_vox(const int4* __restrict__ 
                                                        const uint32_t* __restrict__ bricks,
                                                        uint32_t* __restrict__ nbr, int32_t* __restrict__ gray,
                                                        uint32_t* __restrict__ bin, const uint32_t* __restrict__ ndev,
-                                                       uint32_t* __restrict__ cnt0, int ntiles, int tile_keys) {
+                                                       uint32_t* __restrict__ cnt0, int tile_keys) {
   __shared__ uint32_t rows[NVV * 27];
   __shared__ uint32_t dcnt[512];
   if (ndev) n = min<i64>(n, *ndev);
@@ -267,11 +267,13 @@ __global__ void __launch_bounds__(NVV) k_neighbors_vox(const int4* __restrict__ 
   }
   __syncthreads();
   // the sort's first pass counts its tiles' low 9-bit digits: this workgroup's voxels all lie in tile v0 / tile_keys
-  const i64 tile = v0 / tile_keys;
+  if (cnt0) {
+    uint32_t* tc = cnt0 + v0 / tile_keys * 512;
 #pragma unroll
-  for (int k = 0; k < 2; k++) {
-    const int d = k * NVV + tid;
-    if (dcnt[d]) atomicAdd(&cnt0[(i64)d * ntiles + tile], dcnt[d]);
+    for (int k = 0; k < 2; k++) {
+      const int d = k * NVV + tid;
+      if (dcnt[d]) atomicAdd(&tc[d], dcnt[d]);
+    }
   }
   const int tot = nv * 27;
   uint32_t* o = nbr + v0 * 27;
@@ -384,10 +386,12 @@ SpConvCache build_neighbors_impl(const int4* coords, i64 n, const uint32_t* ndev
     k_brick_mask<<<1, 1024, 0, s>>>(part.ptr<uint32_t>(), nb, cap, maskp, ndev, 4);
   }
   // the sort's workspace: its first pass is counted by the neighbour kernel (slots and counts zeroed with the table)
-  SortWork sw = sort_work(n, 27);
+  // (a device-side count: children of a subdivision, 35-50% of the capacity of 8 per parent; tiles for the capacity of
+  // 4.8 M left 1.7 M children 410 of them: subdivision, map and conv 1094 -> 1084 us)
+  SortWork sw = sort_work(n, 27, ndev ? n / 8 * 3 : n);
   REQ((sw.rch * 256) % NVV == 0, "sort tile of %d keys", sw.rch * 256);
   k_table_clear<<<(int)std::min<i64>(cdiv(std::max<i64>((i64)cap, sw.zwords), 256), 4096), 256, 0, s>>>(
-      t, mask0, maskp, sw.buf.ptr<uint32_t>(), sw.zwords);
+      t, mask0, maskp, (uint32_t*)sw.buf.p, sw.zwords);
   // at most n occupied bricks: the table (capacity >= 2n) never fills. Brick records are indexed by the row of
   // the voxel that inserted the brick, so the record array has n slots (only occupied bricks' records are touched).
   Tensor bricks = empty({n * 64}, I32);
@@ -395,7 +399,7 @@ SpConvCache build_neighbors_impl(const int4* coords, i64 n, const uint32_t* ndev
   k_brick_fill<<<cdiv(n, 256), 256, 0, s>>>(coords, n, W4, H4, D4, t, mask0, maskp, bricks.ptr<uint32_t>(), ndev);
   k_neighbors_vox<<<cdiv(n, NVV), NVV, 0, s>>>(coords, n, W, H, D, t, mask0, maskp, bricks.ptr<uint32_t>(),
                                                c.nbr.ptr<uint32_t>(), c.gray.ptr<int32_t>(), bin.ptr<uint32_t>(),
-                                               ndev, sw.counts(), sw.ntiles, sw.rch * 256);
+                                               ndev, sw.counts(), sw.rch * 256);
   CK(hipGetLastError());
   stable_argsort27(bin.ptr<uint32_t>(), n, c.sorted.ptr<int32_t>(), ndev, &sw);
   c.W = W;

@@ -10,15 +10,17 @@ void excl_scan_u32_ws(const uint32_t* in, uint32_t* out, i64 n, uint32_t* total_
 
 // Workspace of the radix sort (9-bit digits, tiles of 256 * rch keys). A producer of the keys may count the first
 // pass itself: it zeroes the first `zwords` u32 of `buf` beforehand (digit-sum slots, then the first pass's counts)
-// and adds, for each key i of the first n, one to counts[(key_i & 511) * ntiles + i / (256 * rch)], the counts
+// and adds, for each key i of the first n, one to counts[i / (256 * rch) * 512 + (key_i & 511)], the counts
 // starting at u32 word `passes * 1024` of `buf`. Passing the workspace to the sort then skips the first count kernel.
+// Few keys are sorted by passes that count for themselves: rch is 0 and there is nothing to zero or to count.
 struct SortWork {
   int passes = 0, rch = 0, ntiles = 0;
   i64 zwords = 0;
   Tensor buf;
-  uint32_t* counts() const { return buf.ptr<uint32_t>() + (i64)passes * 1024; }
+  uint32_t* counts() const { return rch == 0 ? nullptr : buf.ptr<uint32_t>() + (i64)passes * 1024; }
 };
-SortWork sort_work(i64 n, int bits);
+// likely: the key count to pick the tile size for, where n is a capacity.
+SortWork sort_work(i64 n, int bits, i64 likely);
 
 // Stable ascending argsort of 27-bit keys: order[k] = row index of the k-th smallest key, ties in row order.
 // ndev (device u32, optional): the number of keys, when n is only a capacity bound known to the host.

@@ -2,12 +2,14 @@
 // permutation (src/spconv.cu:47-52: cub::DeviceRadixSort::SortPairs(bin -> iota), stable, bits 0..32; bin < 2^27
 // so bits 27..31 are all zero and sorting 27 bits gives the same order).
 //
-// Three launches per pass over tiles of 256 x RCH keys (RCH = 4, 8 or 16, so there are at least ~900 tiles when
+// Up to kSmallKeys keys: one launch per pass (k_rs_pass).
+// More: three launches per pass over tiles of 256 x RCH keys (RCH = 4, 8 or 16, so there are at least ~900 tiles when
 // the input allows it):
-//   count      : per-tile digit counts, digit-major [512][ntiles] (the first one also zeroes the digit-sum slots;
-//                a producer that already holds the keys may count the first pass itself, see SortWork)
-//   digit scan : one workgroup per digit sums its row and publishes the sum; its start is the sum of the lower
-//                digits' published sums (read back all at once); the row is scanned to exclusive tile starts.
+//   count      : per-tile digit counts, tile-major [ntiles][512], so that a tile's counts are whole lines (the first
+//                one also zeroes the digit-sum slots; a producer that already holds the keys may count the first pass
+//                itself, see SortWork)
+//   digit scan : one workgroup per 16 digits sums their columns and publishes the sums; a digit's start is the sum of
+//                the lower digits' published sums (read back all at once); the columns become exclusive tile starts.
 //                One launch instead of a device-wide scan's three.
 //   scatter    : each wavefront ranks its chunks of 64 keys in order; within a chunk, lanes holding the same digit
 //                find each other with 9 ballots (one per digit bit) and take rank = popcount(peers below me);
@@ -54,7 +56,7 @@ __device__ __forceinline__ void rank_chunks(const uint32_t* __restrict__ kin, co
 // first digit scan reads them), which saves the sort a launch.
 template <int RCH>
 __global__ void __launch_bounds__(RT) k_rs_count(const uint32_t* __restrict__ keys, i64 n, int shift,
-                                                 uint32_t* __restrict__ hist, int ntiles, uint32_t* __restrict__ zero,
+                                                 uint32_t* __restrict__ hist, uint32_t* __restrict__ zero,
                                                  int zn, const uint32_t* __restrict__ ndev) {
   __shared__ uint32_t cnt[NBUK];
   if (ndev) {  // device-side key count: tiles past it are skipped (the digit scan reads only the tiles below it)
@@ -72,13 +74,13 @@ __global__ void __launch_bounds__(RT) k_rs_count(const uint32_t* __restrict__ ke
     if (i < n) atomicAdd(&cnt[(keys[i] >> shift) & (NBUK - 1)], 1u);
   }
   __syncthreads();
-  for (int d = threadIdx.x; d < NBUK; d += RT) hist[(i64)d * ntiles + blockIdx.x] = cnt[d];
+  for (int d = threadIdx.x; d < NBUK; d += RT) hist[(i64)blockIdx.x * NBUK + d] = cnt[d];
 }
 
 template <int RCH>
 __global__ void __launch_bounds__(RT) k_rs_scatter(const uint32_t* __restrict__ kin, const int32_t* __restrict__ vin,
                                                    uint32_t* __restrict__ kout, int32_t* __restrict__ vout, i64 n,
-                                                   int shift, const uint32_t* __restrict__ start, int ntiles,
+                                                   int shift, const uint32_t* __restrict__ start,
                                                    const uint32_t* __restrict__ ndev) {
   __shared__ uint32_t cnt[RT / 64][NBUK];
   if (ndev) {
@@ -95,7 +97,7 @@ __global__ void __launch_bounds__(RT) k_rs_scatter(const uint32_t* __restrict__ 
   rank_chunks<RCH>(kin, vin, n, shift, seg, lane, cnt[wv], key, val, rank);
   __syncthreads();
   for (int d = threadIdx.x; d < NBUK; d += RT) {
-    uint32_t run = start[(i64)d * ntiles + blockIdx.x];
+    uint32_t run = start[(i64)blockIdx.x * NBUK + d];
 #pragma unroll
     for (int w = 0; w < RT / 64; w++) {
       uint32_t t = cnt[w][d];
@@ -116,87 +118,158 @@ __global__ void __launch_bounds__(RT) k_rs_scatter(const uint32_t* __restrict__ 
   }
 }
 
-// Per-pass tile starts in one launch: workgroup d owns digit d. It sums its row of per-tile counts (digit-major,
-// [NBUK][ntiles]) and publishes the sum (flag in the high word of a zeroed 64-bit slot); the digit's start is the
-// sum of the lower digits' published sums, read back all at once (workgroups start in id order, so every lower
-// digit's workgroup is already running and publishes without waiting). The wait is bounded: a sum not published
-// within spin_limit polls is computed by the waiting workgroup from that digit's row of tile counts, so the
-// result never depends on the schedule (the limit only trades waiting against re-reading). The row is then
-// scanned to exclusive tile starts in `start` (not in place: the counts stay intact for such a fallback read).
-__global__ void __launch_bounds__(RT) k_rs_digit_scan(const uint32_t* __restrict__ cnt,
-                                                      uint32_t* __restrict__ start, uint64_t* __restrict__ dsum,
-                                                      int ntiles, uint32_t spin_limit, const uint32_t* __restrict__ ndev,
-                                                      int tile_keys) {
-  __shared__ uint32_t red[RT / 64];
-  const int d = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-  const int stride = ntiles;  // rows keep the capacity stride
-  const uint32_t* row = cnt + (i64)d * stride;
-  uint32_t* orow = start + (i64)d * stride;
+// Per-pass tile starts in one launch: workgroup b owns digits 16 b .. +16, and its thread (tile group g of 64, digit)
+// a run of consecutive tiles. Column sums give each digit's total, which is published (flag in the high word of a zeroed
+// 64-bit slot); the digit's start is the sum of the lower digits' published totals, read back all at once (workgroups
+// start in id order, so every lower digit's workgroup is already running and publishes without waiting). The wait is
+// bounded: a total not published within spin_limit polls is summed by the waiting lane from the tile counts, so the
+// result never depends on the schedule (the limit only trades waiting against re-reading). The columns then become
+// exclusive tile starts in `start` (not in place: the counts stay intact for such a fallback read).
+// It is bound by its dependent round trips, not by bytes. With digit-major counts and one workgroup per digit, every
+// tile's 512 counts and starts were 512 separate lines, for the count and the scatter kernel too: 1.2 M keys, count
+// 10.3 -> 6.6 us, scan 10.8 -> 9.2, scatter 10.8 -> 9.2.
+constexpr int DPW = 16, TG = 64, HELD = 32;  // digits per workgroup, tile groups, counts held by a thread
+__global__ void __launch_bounds__(DPW* TG) k_rs_digit_scan(const uint32_t* __restrict__ cnt,
+                                                           uint32_t* __restrict__ start, uint64_t* __restrict__ dsum,
+                                                           int ntiles, uint32_t spin_limit,
+                                                           const uint32_t* __restrict__ ndev, int tile_keys) {
+  __shared__ uint32_t part[DPW][TG + 1], tot[DPW], low[DPW];
+  const int d0 = blockIdx.x * DPW, tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
   if (ndev) ntiles = max(1, min(ntiles, (int)(((i64)*ndev + tile_keys - 1) / tile_keys)));  // tiles with keys
-  auto wg_sum = [&](uint32_t v) __attribute__((always_inline)) {
+  const int dd = tid % DPW, g = tid / DPW, per = (ntiles + TG - 1) / TG;
+  const int t0 = min(g * per, ntiles), t1 = min(t0 + per, ntiles);
+  const uint32_t* col = cnt + d0 + dd;
+  uint32_t mine = 0, c[HELD];  // a short run is read once, all of it in flight, and held; a long one read twice
+  const bool held = per <= HELD;
+  if (held) {
 #pragma unroll
-    for (int o = 32; o >= 1; o >>= 1) v += (uint32_t)__shfl_xor((int)v, o, 64);
-    if (lane == 0) red[wv] = v;
-    __syncthreads();
-    uint32_t all = 0;
+    for (int k = 0; k < HELD; k++) c[k] = t0 + k < t1 ? col[(i64)(t0 + k) * NBUK] : 0u;
 #pragma unroll
-    for (int w = 0; w < RT / 64; w++) all += red[w];
-    __syncthreads();
-    return all;
-  };
-  uint32_t mine = 0;
-  for (int i = tid; i < ntiles; i += RT) mine += row[i];
-  const uint32_t rsum = wg_sum(mine);
-  if (tid == 0) __hip_atomic_store(dsum + d, ST_SUM | rsum, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    for (int k = 0; k < HELD; k++) mine += c[k];
+  } else {
+#pragma unroll 8
+    for (int t = t0; t < t1; t++) mine += col[(i64)t * NBUK];
+  }
+  part[dd][g] = mine;
+  __syncthreads();
+  static_assert(DPW == 16 && TG == 64 && NBUK <= DPW * TG, "one wavefront per digit, one published sum per thread");
+  // wavefront wv: digit d0 + wv, lane = tile group
+  const uint32_t v = part[wv][lane];
+  uint32_t inc = v;
+#pragma unroll
+  for (int o = 1; o < 64; o <<= 1) {
+    const uint32_t t = (uint32_t)__shfl_up((int)inc, o, 64);
+    if (lane >= o) inc += t;
+  }
+  if (lane == 63) {
+    __hip_atomic_store(dsum + d0 + wv, ST_SUM | inc, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    tot[wv] = inc;
+  }
   uint32_t below = 0;
-  for (int e = tid; e < d; e += RT) {
-    uint64_t w = __hip_atomic_load(dsum + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  if (tid < d0) {  // the digits of the lower workgroups, one per thread
+    uint64_t w = __hip_atomic_load(dsum + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     for (uint32_t spins = 0; (w >> 32) == 0 && spins < spin_limit; spins++)
-      w = __hip_atomic_load(dsum + e, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      w = __hip_atomic_load(dsum + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if ((w >> 32) == 0) {
-      // not published within the limit: sum digit e's row of tile counts here (they are complete: the count
-      // kernel ran before this launch), so the start is exact whatever the workgroup schedule
+      // not published within the limit: sum the digit's tile counts here (they are complete: the count kernel ran
+      // before this launch), so the start is exact whatever the workgroup schedule
       uint32_t s = 0;
-      for (int i = 0; i < ntiles; i++) s += cnt[(i64)e * stride + i];
+      for (int t = 0; t < ntiles; t++) s += cnt[(i64)t * NBUK + tid];
       w = s;
     }
-    below += (uint32_t)w;
+    below = (uint32_t)w;
   }
-  uint32_t carry = wg_sum(below);
-  for (int b = 0; b < ntiles; b += RT) {
-    const int i = b + tid;
-    const uint32_t v = i < ntiles ? row[i] : 0u;
-    uint32_t inc = v;
+#pragma unroll
+  for (int o = 32; o >= 1; o >>= 1) below += (uint32_t)__shfl_xor((int)below, o, 64);
+  if (lane == 0) low[wv] = below;
+  __syncthreads();
+  uint32_t first = 0;
+#pragma unroll
+  for (int w = 0; w < DPW; w++) first += low[w] + (w < wv ? tot[w] : 0u);
+  part[wv][lane] = first + inc - v;
+  __syncthreads();
+  uint32_t run = part[dd][g];
+  uint32_t* out = start + d0 + dd;
+  if (held) {
+#pragma unroll
+    for (int k = 0; k < HELD; k++) {
+      if (t0 + k < t1) out[(i64)(t0 + k) * NBUK] = run;
+      run += c[k];
+    }
+    return;
+  }
+#pragma unroll 8
+  for (int t = t0; t < t1; t++) {
+    const uint32_t v = col[(i64)t * NBUK];
+    out[(i64)t * NBUK] = run;
+    run += v;
+  }
+}
+
+// One pass in one launch, for few keys: every workgroup (1024 keys, one chunk per wavefront) counts the digits of all
+// n keys itself, those of the tiles before its own apart, which gives its tile starts without a count and a scan
+// launch; ranks and destinations are the scatter kernel's.
+__global__ void __launch_bounds__(1024) k_rs_pass(const uint32_t* __restrict__ kin, const int32_t* __restrict__ vin,
+                                                  uint32_t* __restrict__ kout, int32_t* __restrict__ vout, int n,
+                                                  int shift, const uint32_t* __restrict__ ndev) {
+  constexpr int NW = 16;
+  __shared__ uint32_t cnt[NW][NBUK], before[NBUK], rest[NBUK], red[NBUK / 64];
+  if (ndev) n = min((uint32_t)n, *ndev);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, base = blockIdx.x * 1024;
+  if (base >= n) return;
+  for (int d = lane; d < NBUK; d += 64) cnt[wv][d] = 0;
+  if (tid < NBUK) before[tid] = rest[tid] = 0;
+  __syncthreads();
+#pragma unroll 4
+  for (int i = tid; i < n; i += 1024) atomicAdd(&(i < base ? before : rest)[(kin[i] >> shift) & (NBUK - 1)], 1u);
+  uint32_t key[1], rank[1];
+  int32_t val[1];
+  rank_chunks<1>(kin, vin, n, shift, base + wv * 64, lane, cnt[wv], key, val, rank);
+  __syncthreads();
+  uint32_t tot = 0, inc = 0;
+  if (tid < NBUK) {
+    inc = tot = before[tid] + rest[tid];
 #pragma unroll
     for (int o = 1; o < 64; o <<= 1) {
       const uint32_t t = (uint32_t)__shfl_up((int)inc, o, 64);
       if (lane >= o) inc += t;
     }
     if (lane == 63) red[wv] = inc;
-    __syncthreads();
-    uint32_t base = carry, all = 0;
+  }
+  __syncthreads();
+  if (tid < NBUK) {
+    uint32_t run = inc - tot + before[tid];
 #pragma unroll
-    for (int w = 0; w < RT / 64; w++) {
-      const uint32_t t = red[w];
-      if (w < wv) base += t;
-      all += t;
+    for (int w = 0; w < NBUK / 64; w++) run += w < wv ? red[w] : 0u;
+#pragma unroll
+    for (int w = 0; w < NW; w++) {
+      const uint32_t t = cnt[w][tid];
+      cnt[w][tid] = run;
+      run += t;
     }
-    if (i < ntiles) orow[i] = base + inc - v;
-    carry += all;
-    __syncthreads();
+  }
+  __syncthreads();
+  if (base + tid < n) {
+    const uint32_t pos = cnt[wv][(key[0] >> shift) & (NBUK - 1)] + rank[0];
+    if (kout) kout[pos] = key[0];  // the last pass writes only the values
+    vout[pos] = val[0];
   }
 }
+// Kernel map and quads of n voxels, one launch per pass / three: 8000 44 / 62 us, 15000 52 / 63, 20000 58 / 64, 30000
+// 70 / 64, 60000 115 / 66: counting all keys in every workgroup pays up to ~24 k of them.
+constexpr i64 kSmallKeys = 1024 * 24;
 }  // namespace
 
-SortWork sort_work(i64 n, int bits) {
+SortWork sort_work(i64 n, int bits, i64 likely) {
   SortWork w;
   w.passes = (bits + RBITS - 1) / RBITS;
+  if (n <= kSmallKeys) return w;  // each pass counts for itself: no workspace, nothing to count
   // the largest tile that still leaves ~900 tiles (interleaved builds, one box: C3 0.390 M keys best at 4, C4 3.76 M
   // at 16 (8: +3%), C5's children 2.15 M at 8 (16: +1.2%))
-  w.rch = n >= (i64)RT * 16 * 900 ? 16 : (n >= (i64)RT * 8 * 900 ? 8 : 4);
+  w.rch = likely >= (i64)RT * 16 * 900 ? 16 : (likely >= (i64)RT * 8 * 900 ? 8 : 4);
   w.ntiles = (int)std::max<i64>(cdiv(n, (i64)RT * w.rch), 1);
   w.zwords = (i64)w.passes * NBUK * 2 + (i64)NBUK * w.ntiles;
-  // [digit-sum slots: passes x NBUK u64][first pass's counts: NBUK x ntiles][tile starts: NBUK x ntiles]; the
+  // [digit-sum slots: passes x NBUK u64][first pass's counts: ntiles x NBUK][tile starts: ntiles x NBUK]; the
   // slot words are even in number, so the 64-bit slots and everything after them stay 8-byte aligned
   w.buf = empty({w.zwords + (i64)NBUK * w.ntiles}, I32);
   return w;
@@ -212,10 +285,12 @@ void stable_sort_pairs(const uint32_t* keys, const int32_t* vals, i64 n, int bit
   // itself; the tests use it to check that path)
   uint32_t spin_limit = kSpinLimit;
   if (const char* e = getenv("SPCONV_SORT_SPIN_LIMIT")) spin_limit = (uint32_t)strtoul(e, nullptr, 10);
+  const bool small = n <= kSmallKeys;
   SortWork own;
-  if (!pre) own = sort_work(n, bits);
+  if (!pre) own = sort_work(n, bits, n);
   SortWork& w = pre ? *pre : own;
-  REQ(w.passes == (bits + RBITS - 1) / RBITS && w.ntiles == (int)std::max<i64>(cdiv(n, (i64)RT * w.rch), 1),
+  REQ(w.passes == (bits + RBITS - 1) / RBITS &&
+          (small ? w.rch == 0 : w.ntiles == (int)std::max<i64>(cdiv(n, (i64)RT * w.rch), 1)),
       "sort workspace made for another size");
   const int passes = w.passes, rch = w.rch, ntiles = w.ntiles;
   Tensor kb0 = empty({n}, I32), kb1 = empty({n}, I32), vb0 = empty({n}, I32), vb1 = empty({n}, I32);
@@ -226,6 +301,18 @@ void stable_sort_pairs(const uint32_t* keys, const int32_t* vals, i64 n, int bit
     kout = p + 1 == passes ? nullptr : ((p & 1) ? kb1.ptr<uint32_t>() : kb0.ptr<uint32_t>());
     vout = p + 1 == passes ? vals_out : ((p & 1) ? vb1.ptr<int32_t>() : vb0.ptr<int32_t>());
   };
+  if (small) {
+    for (int p = 0; p < passes; p++) {
+      uint32_t* kout;
+      int32_t* vout;
+      outs(p, kout, vout);
+      k_rs_pass<<<cdiv(n, 1024), 1024, 0, s>>>(kin, vin, kout, vout, (int)n, p * RBITS, ndev);
+      kin = kout;
+      vin = vout;
+    }
+    CK(hipGetLastError());
+    return;
+  }
   const i64 swords = (i64)passes * NBUK * 2;
   uint64_t* dsum = (uint64_t*)w.buf.ptr<uint32_t>();
   uint32_t* h = w.buf.ptr<uint32_t>() + swords;
@@ -238,14 +325,14 @@ void stable_sort_pairs(const uint32_t* keys, const int32_t* vals, i64 n, int bit
     if (p > 0 || !pre) {  // a caller-made workspace arrives with the first pass counted and the slots zeroed
       uint32_t* z = p == 0 ? (uint32_t*)dsum : nullptr;  // the first count kernel zeroes every pass's digit sums
       const int zn = (int)swords;
-      if (rch == 16) k_rs_count<16><<<ntiles, RT, 0, s>>>(kin, n, shift, h, ntiles, z, zn, ndev);
-      else if (rch == 8) k_rs_count<8><<<ntiles, RT, 0, s>>>(kin, n, shift, h, ntiles, z, zn, ndev);
-      else k_rs_count<4><<<ntiles, RT, 0, s>>>(kin, n, shift, h, ntiles, z, zn, ndev);
+      if (rch == 16) k_rs_count<16><<<ntiles, RT, 0, s>>>(kin, n, shift, h, z, zn, ndev);
+      else if (rch == 8) k_rs_count<8><<<ntiles, RT, 0, s>>>(kin, n, shift, h, z, zn, ndev);
+      else k_rs_count<4><<<ntiles, RT, 0, s>>>(kin, n, shift, h, z, zn, ndev);
     }
-    k_rs_digit_scan<<<NBUK, RT, 0, s>>>(h, st, dsum + p * NBUK, ntiles, spin_limit, ndev, RT * rch);
-    if (rch == 16) k_rs_scatter<16><<<ntiles, RT, 0, s>>>(kin, vin, kout, vout, n, shift, st, ntiles, ndev);
-    else if (rch == 8) k_rs_scatter<8><<<ntiles, RT, 0, s>>>(kin, vin, kout, vout, n, shift, st, ntiles, ndev);
-    else k_rs_scatter<4><<<ntiles, RT, 0, s>>>(kin, vin, kout, vout, n, shift, st, ntiles, ndev);
+    k_rs_digit_scan<<<NBUK / DPW, DPW * TG, 0, s>>>(h, st, dsum + p * NBUK, ntiles, spin_limit, ndev, RT * rch);
+    if (rch == 16) k_rs_scatter<16><<<ntiles, RT, 0, s>>>(kin, vin, kout, vout, n, shift, st, ndev);
+    else if (rch == 8) k_rs_scatter<8><<<ntiles, RT, 0, s>>>(kin, vin, kout, vout, n, shift, st, ndev);
+    else k_rs_scatter<4><<<ntiles, RT, 0, s>>>(kin, vin, kout, vout, n, shift, st, ndev);
     kin = kout;
     vin = vout;
   }
