@@ -332,20 +332,22 @@ __global__ void k_c2s_count(const uint4* __restrict__ lg, i64 n, uint32_t* __res
   cnt[i] = c;
 }
 
-__global__ void k_c2s_emit(const uint4* __restrict__ lg, const int4* __restrict__ co, const uint32_t* __restrict__ off,
-                           i64 n, int4* __restrict__ nco, int32_t* __restrict__ src) {
-  i64 i = (i64)blockIdx.x * blockDim.x + threadIdx.x;
+// One lane per (parent, slot): a kept slot's place is the parent's offset plus the kept slots below it in the parent's
+// 8 lanes, so a wavefront's children leave as one contiguous range. One thread per parent stored its children one by
+// one, 20 bytes at a time: 301 k parents, 1.2 M children 18.8 us against 11.5 (600 k parents, 1.7 M children: 21.4 / 19.1).
+__global__ void __launch_bounds__(256) k_c2s_emit(const uint16_t* __restrict__ lg, const int4* __restrict__ co,
+                                                  const uint32_t* __restrict__ off, i64 n, int4* __restrict__ nco,
+                                                  int32_t* __restrict__ src) {
+  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x, i = e >> 3;
   if (i >= n) return;
-  uint4 q = lg[i];
-  uint32_t w[4] = {q.x, q.y, q.z, q.w}, r = off[i];
-  int4 p = co[i];
-#pragma unroll
-  for (int s = 0; s < 8; s++)
-    if (f16_positive((w[s >> 1] >> ((s & 1) * 16)) & 0xffffu)) {
-      nco[r] = make_int4(p.x, p.y * 2 + (s & 1), p.z * 2 + (s >> 1 & 1), p.w * 2 + (s >> 2 & 1));
-      src[r] = (int32_t)(i * 8 + s);
-      r++;
-    }
+  const int s = threadIdx.x & 7, lane = threadIdx.x & 63;
+  const bool keep = f16_positive(lg[e]);
+  const uint32_t kept = (uint32_t)(__ballot(keep) >> (lane & ~7)) & 0xffu;
+  if (!keep) return;
+  const uint32_t r = off[i] + __popc(kept & ((1u << s) - 1u));
+  const int4 p = co[i];
+  nco[r] = make_int4(p.x, p.y * 2 + (s & 1), p.z * 2 + (s >> 1 & 1), p.w * 2 + (s >> 2 & 1));
+  src[r] = (int32_t)e;
 }
 }  // namespace
 
@@ -842,7 +844,7 @@ Subdivision subdivide(const Tensor& coords, const Tensor& logits) {
   o.coords = empty({m, 4}, I32);
   o.src = empty({m}, I32);
   if (m) {
-    k_c2s_emit<<<cdiv(n, 256), 256, 0, s>>>(logits.ptr<uint4>(), coords.ptr<int4>(), off.ptr<uint32_t>(), n,
+    k_c2s_emit<<<cdiv(8 * n, 256), 256, 0, s>>>(logits.ptr<uint16_t>(), coords.ptr<int4>(), off.ptr<uint32_t>(), n,
                                             o.coords.ptr<int4>(), o.src.ptr<int32_t>());
     CK(hipGetLastError());
   }
@@ -894,7 +896,7 @@ UpsampleLevel subdivide_build(const Tensor& coords, const Tensor& logits, int W,
   CountReadback& rb = count_readback();
   CK(hipMemcpyAsync(rb.host, mdev, sizeof(uint32_t), hipMemcpyDeviceToHost, s));
   CK(hipEventRecord(rb.ev, s));
-  k_c2s_emit<<<cdiv(n, 256), 256, 0, s>>>(logits.ptr<uint4>(), coords.ptr<int4>(), off.ptr<uint32_t>(), n,
+  k_c2s_emit<<<cdiv(8 * n, 256), 256, 0, s>>>(logits.ptr<uint16_t>(), coords.ptr<int4>(), off.ptr<uint32_t>(), n,
                                           cc.ptr<int4>(), src.ptr<int32_t>());
   CK(hipGetLastError());
   // the children's map, sized for the capacity and stopped at the device-side count by every kernel
@@ -966,7 +968,7 @@ void subdivide_noalloc(const int32_t* coords, const uint16_t* logits_f16, i64 n,
   k_c2s_count<<<cdiv(n + 1, 256), 256, 0, s>>>((const uint4*)logits_f16, n, off);
   excl_scan_u32_ws(off, off, n + 1, nullptr, part);
   k_store_count<<<1, 64, 0, s>>>(off + n, m_dev);
-  k_c2s_emit<<<cdiv(n, 256), 256, 0, s>>>((const uint4*)logits_f16, (const int4*)coords, off, n, (int4*)child_coords,
+  k_c2s_emit<<<cdiv(8 * n, 256), 256, 0, s>>>(logits_f16, (const int4*)coords, off, n, (int4*)child_coords,
                                           src);
   CK(hipGetLastError());
 }
