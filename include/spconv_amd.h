@@ -58,6 +58,8 @@ int spc_cache_lookup(const spc_cache* c, const int32_t* query, int64_t m, int32_
  * built over one batch with W = H = D = R.
  * Replaces: k_fdg_quads and its hash (src/mesh.cu:7-19, 36-45, 54-62). */
 int spc_fdg_quads(const spc_cache* c, const float* h, int32_t* quad, int32_t* ok);
+/* The same with quad[e] = -1 where ok[e] = 0: the buffer needs no fill beforehand. */
+int spc_fdg_quads_filled(const spc_cache* c, const float* h, int32_t* quad, int32_t* ok);
 
 /* Trilinear sample map of L points grid f32 [L,3] (continuous voxel coordinates: voxel i spans [i, i+1)) in batch
  * `batch` of a cache built with SPC_KEEP_HASH: nb u32 [L,8] = the rows of the 8 voxels around p - 0.5 (corner

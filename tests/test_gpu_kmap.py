@@ -293,6 +293,23 @@ def test_grid_sample(gpu, name):
     assert bool((nb3 == -1).all()) and bool((wt3 == 0).all())
 
 
+def test_fdg_quads_fill(gpu):
+    """spc_fdg_quads leaves the quads of edges without one untouched; spc_fdg_quads_filled, which fdg_quads calls on
+    uninitialised memory, sets them to -1; flags and the other quads are the same."""
+    import ctypes
+    c = coords("c1")
+    h = torch.from_numpy(np.random.default_rng(4).standard_normal((len(c), 7)).astype(np.float32)).to(gpu)
+    cache = sp.build_neighbors(torch.from_numpy(c).to(gpu), 32, 32, 32)
+    quad, ok = sp.fdg_quads(cache, h)
+    keep = torch.full_like(quad, 77)
+    ok2 = torch.empty_like(ok)
+    p = lambda t: ctypes.c_void_p(t.data_ptr())
+    assert sp.load_library().spc_fdg_quads(cache._h, p(h), p(keep), p(ok2)) == 0
+    has = ok > 0
+    assert torch.equal(ok, ok2) and 0 < int(has.sum()) < len(ok)
+    assert torch.equal(quad[has], keep[has]) and bool((quad[~has] == -1).all()) and bool((keep[~has] == 77).all())
+
+
 @pytest.mark.parametrize("L", [1, 31, 32, 33, 63, 65, 4000])
 def test_grid_sample_ragged(gpu, L):
     """Point counts around the sample map's 64-point workgroup, points that are not finite among them: rows and

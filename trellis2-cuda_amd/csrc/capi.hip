@@ -73,14 +73,23 @@ SPC_API int spc_cache_lookup(const spc_cache* c, const int32_t* query, int64_t m
   });
 }
 
-SPC_API int spc_fdg_quads(const spc_cache* c, const float* h, int32_t* quad, int32_t* ok) {
+namespace {
+int fdg_quads_c(const spc_cache* c, const float* h, int32_t* quad, int32_t* ok, bool fill) {
   return guarded([&] {
     REQ(c, "cache is null");
     const i64 n = c->c.N;
     REQ(n == 0 || (h && quad && ok), "null h/quad/ok");
     Tensor tq = borrow(quad, {3 * n, 4}, I32), to = borrow(ok, {3 * n}, I32);
-    fdg_quads(c->c, borrow(h, {n, 7}, F32), tq, to);
+    const Tensor th = borrow(h, {n, 7}, F32);
+    fill ? fdg_quads_filled(c->c, th, tq, to) : fdg_quads(c->c, th, tq, to);
   });
+}
+}  // namespace
+SPC_API int spc_fdg_quads(const spc_cache* c, const float* h, int32_t* quad, int32_t* ok) {
+  return fdg_quads_c(c, h, quad, ok, false);
+}
+SPC_API int spc_fdg_quads_filled(const spc_cache* c, const float* h, int32_t* quad, int32_t* ok) {
+  return fdg_quads_c(c, h, quad, ok, true);
 }
 
 SPC_API int spc_cache_free(spc_cache* c) {

@@ -95,10 +95,12 @@ void grid_sample_sum(const Tensor& x, const Tensor& nb, const Tensor& wt, Tensor
 
 // FlexiDualGrid quads from the kernel map, no hash probes (reference k_fdg_quads, src/mesh.cu:36-45): for voxel i
 // and axis a (e = 3i + a), if h[i,3+a] > 0 and the 4 voxels at the axis' edge offsets (all inside the 3x3x3
-// neighbourhood) exist, ok[e] = 1 and quad[e] = their rows, else ok[e] = 0 (quad[e] left untouched). h f32 [N,7],
+// neighbourhood) exist, ok[e] = 1 and quad[e] = their rows, else ok[e] = 0 (quad[e] left untouched; -1 in
+// fdg_quads_filled). h f32 [N,7],
 // quad int32 [3N,4], ok int32 [3N]. Equal to the reference when the cache was built with W = H = D = R over one
 // batch (the reference's mesh hash key ignores the batch).
 void fdg_quads(const SpConvCache& c, const Tensor& h, Tensor& quad, Tensor& ok);
+void fdg_quads_filled(const SpConvCache& c, const Tensor& h, Tensor& quad, Tensor& ok);
 
 // Tile choice. The reference replays FlexGEMM's autotune table (src/spconv.cu:177-221); here the tile is fixed
 // per channel width (B1 = rows per tile and per schedule block, BK = channels per K stage, S = 1).

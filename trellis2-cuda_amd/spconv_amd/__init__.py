@@ -26,7 +26,7 @@ EMPTY = 0xFFFFFFFF
 
 # the C ABI's exported symbols (every declaration of include/spconv_amd.h)
 SYMBOLS = ("spc_last_error", "spc_set_stream", "spc_build_neighbors", "spc_build_neighbors_ex", "spc_cache_lookup",
-           "spc_fdg_quads", "spc_cache_free", "spc_cache_info", "spc_cache_valid", "spc_conv_cfg",
+           "spc_fdg_quads", "spc_fdg_quads_filled", "spc_cache_free", "spc_cache_info", "spc_cache_valid", "spc_conv_cfg",
            "spc_conv_cfg_autotune", "spc_conv_cfg_autotune_strict", "spc_subm_conv", "spc_subm_conv_fused", "spc_subm_conv_gathered",
            "spc_gather_ln_act", "spc_add_skip", "spc_convnext_mlp", "spc_subm_conv_skip",
            "spc_subdivide", "spc_subdivide_noalloc", "spc_subm_conv_replay", "spc_grid_sample_map",
@@ -53,6 +53,7 @@ def load_library():
     L.spc_build_neighbors_ex.argtypes = [P, I64, I, I, I, I, PP]
     L.spc_cache_lookup.argtypes = [P, P, I64, P]
     L.spc_fdg_quads.argtypes = [P, P, P, P]
+    L.spc_fdg_quads_filled.argtypes = [P, P, P, P]
     L.spc_cache_free.argtypes = [P]
     L.spc_cache_info.argtypes = [P, ctypes.POINTER(I64), PP, PP, PP]
     L.spc_cache_valid.argtypes = [P, I, PP, PP, ctypes.POINTER(I64)]
@@ -208,13 +209,13 @@ def lookup(cache: SpConvCache, query):
 
 def fdg_quads(cache: SpConvCache, h):
     """FlexiDualGrid quads from the kernel map (reference k_fdg_quads, src/mesh.cu:36-45): returns (quad int32
-    [3N,4], ok int32 [3N]); quad rows of edges with ok = 0 are unspecified."""
+    [3N,4], ok int32 [3N]); quad rows of edges with ok = 0 are -1."""
     torch = _torch()
     if h.dtype != torch.float32 or h.dim() != 2 or h.shape != (cache.N, 7):
         raise ValueError(f"h must be float32 [{cache.N},7]")
-    quad = torch.full((3 * cache.N, 4), -1, dtype=torch.int32, device=h.device)
+    quad = torch.empty((3 * cache.N, 4), dtype=torch.int32, device=h.device)
     ok = torch.empty(3 * cache.N, dtype=torch.int32, device=h.device)
-    _check(load_library().spc_fdg_quads(cache._h, _ptr(h), _ptr(quad), _ptr(ok)))
+    _check(load_library().spc_fdg_quads_filled(cache._h, _ptr(h), _ptr(quad), _ptr(ok)))
     return quad, ok
 
 
