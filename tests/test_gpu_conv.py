@@ -517,6 +517,13 @@ def test_wide_128_splits(gpu, monkeypatch, ci, co, nrows, splits):
         assert differ == splits
 
 
+@pytest.mark.parametrize("bias_dt", ["f16", "bf16"])
+@pytest.mark.parametrize("ci,co", [(64, 64), (128, 64), (32, 64), (64, 128), (256, 256), (128, 192), (1024, 256)])
+def test_bias_16bit(gpu, ci, co, bias_dt):
+    """A 16-bit bias is widened by the weight repack, or by a pass of its own for the kernel without one (192)."""
+    run_case(gpu, shell(9.0), ci, co, in_dt=bias_dt, act=1, bias_dt=bias_dt, seed=ci + co)
+
+
 def test_wide_tail_split_256_f16(gpu, monkeypatch):
     """256 -> 256, fp16, bias + SiLU on the first 80000 rows of the C3 shell: 625 single-channel-tile row tiles,
     79 per XCD (72 on the last), so the last 15 (8) tiles of each XCD are split along K over 4 (8) workgroups on a

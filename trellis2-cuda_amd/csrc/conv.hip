@@ -46,6 +46,13 @@ __device__ __forceinline__ float load_elem(const void* p, i64 i, int dt) {
   uint16_t h = ((const uint16_t*)p)[i];
   return dt == BF16 ? bf16_to_f32(h) : f16_to_f32(h);
 }
+// A 16-bit bias widened to fp32 by the weight repack's first workgroups (dst null: nothing to do), one launch fewer than
+// a pass of its own (~3 us of a call)
+struct BiasCvt {
+  const void* src;
+  int dt;
+  float* dst;
+};
 __device__ __forceinline__ void store_elem(void* p, i64 i, int dt, float v) {
   if (dt == F32) ((float*)p)[i] = v;
   else ((uint16_t*)p)[i] = dt == BF16 ? f32_to_bf16(v) : f32_to_f16(v);
@@ -510,9 +517,10 @@ __device__ __forceinline__ f32x4v mfma16(u32x4 a, u32x4 b, f32x4v c) {
 // With contig set, step m holds channels m*32 + (l >> 4)*8 .. +8 instead (the operand order of a row read as S
 // contiguous 64-byte pieces, one per step).
 __global__ void __launch_bounds__(64) k_pack_w_narrow(const u32x4* __restrict__ w, u32x4* __restrict__ wp, int Co,
-                                                      int Ci, int contig = 0) {
+                                                      int Ci, BiasCvt b, int contig = 0) {
   const int S = Ci / 32, T = Co / 16, lane = threadIdx.x;
   const int m = blockIdx.x, t = blockIdx.y, v = blockIdx.z;
+  if (b.dst && m == 0 && v == 0 && lane < 16) b.dst[t * 16 + lane] = load_elem(b.src, t * 16 + lane, b.dt);
   const int co = t * 16 + (lane & 15), ch = (contig ? m * 4 + (lane >> 4) : (lane >> 4) * S + m) * 8;
   wp[(((i64)v * T + t) * S + m) * 64 + lane] = w[((i64)co * 27 + v) * Ci / 8 + ch / 8];
 }
@@ -2141,10 +2149,13 @@ void launch_w256(ConvArgs a) {
 // A wavefront then fetches a stage's weight fragment with fully coalesced 1 KiB loads.
 // Grid (nkc*2, 27, Co/64) of 256-thread blocks: block (kc*2 + t, v, slice) writes the four 1 KiB blocks
 // j = 0..3 of that (slice, v, kc, t), thread = j*64 + lane; no thread divides.
-__global__ void __launch_bounds__(256) k_pack_w(const u32x4* __restrict__ w, u32x4* __restrict__ wp, int Co, int Ci) {
+__global__ void __launch_bounds__(256) k_pack_w(const u32x4* __restrict__ w, u32x4* __restrict__ wp, int Ci,
+                                                BiasCvt b) {
   const int nkc = Ci / 64, kc = blockIdx.x >> 1, t = blockIdx.x & 1, v = blockIdx.y, slice = blockIdx.z;
   const int j = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int co = slice * 64 + t * 32 + (lane & 31), ch = kc * 64 + (lane >> 5) * 32 + j * 8;
+  if (b.dst && blockIdx.x == 0 && v == 0 && threadIdx.x < 64)
+    b.dst[slice * 64 + lane] = load_elem(b.src, slice * 64 + lane, b.dt);
   wp[((((i64)slice * 27 + v) * nkc + kc) * 2 + t) * 256 + threadIdx.x] = w[((i64)co * 27 + v) * Ci / 8 + ch / 8];
 }
 
@@ -2317,13 +2328,17 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
   if (N == 0) return;
   SpConvCfg cfg = spconv_cfg(N, Ci, Co);
   Tensor bf;
+  BiasCvt bc{};  // a 16-bit bias is widened by the weight repack, or by k_to_f32 where there is none
   if (b) {
     if (b->dt == F32) bf = *b;
     else {
       bf = empty({Co}, F32);
-      k_to_f32<<<cdiv(Co, 256), 256, 0, stream()>>>(b->p, b->dt, Co, bf.ptr<float>());
+      bc = BiasCvt{b->p, b->dt, bf.ptr<float>()};
     }
   }
+  auto widen_bias = [&] {
+    if (bc.dst) k_to_f32<<<cdiv(Co, 256), 256, 0, stream()>>>(bc.src, bc.dt, Co, bc.dst);
+  };
   ConvArgs a{};
   a.x = x.ptr<uint16_t>();
   a.w = w.ptr<uint16_t>();
@@ -2361,7 +2376,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
   else if (Co == 64 && Ci == 128 && halo128_enabled()) ht = &c.halo_table(HaloShape<4>::B, HaloShape<4>::UM);
   if (ht) {  // halo kernel: narrow weight order, the tile's distinct neighbour rows copied to LDS once
     wpack = empty({(i64)Co * 27 * Ci}, x.dt);
-    k_pack_w_narrow<<<dim3(Ci / 32, Co / 16, 27), 64, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci);
+    k_pack_w_narrow<<<dim3(Ci / 32, Co / 16, 27), 64, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci, bc);
     a.w = wpack.ptr<uint16_t>();
     a.hrows = ht->rows.ptr<int32_t>();
     a.hcount = ht->count.ptr<int32_t>();
@@ -2390,7 +2405,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     // four 16-byte pieces 64 bytes apart (32 lines, each half used): C5 children 0.857 -> 0.823 ms
     a.kcontig = Ci == 128;
     k_pack_w_narrow<<<dim3(Ci / 32, Co / 16, 27), 64, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci,
-                                                                     a.kcontig);
+                                                                     bc, a.kcontig);
     a.w = wpack.ptr<uint16_t>();
     const SpConvCache::RowTable& rt = c.row_table(16);
     a.order = rt.order.ptr<int32_t>();
@@ -2404,6 +2419,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     }
   } else if (Co % 256 == 0 && Ci % 32 == 0 && w8_enabled()) {  // 256 x 256 tiles, both operands through LDS
     wpack = empty({(i64)Co * 27 * Ci}, x.dt);
+    widen_bias();
     k_pack_w8<<<dim3(Ci / 32, 27, Co / 256), 256, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Ci);
     a.w = wpack.ptr<uint16_t>();
     const SpConvCache::RowTable& rt = c.row_table(-1);
@@ -2414,6 +2430,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     a.tsched = c.tile_schedule(-1, 256).ptr<int32_t>();
   } else if (Co % 256 == 0 && Ci % 64 == 0 && w256_enabled()) {  // 256 x 256 tiles: 4 KB weight blocks
     wpack = empty({(i64)Co * 27 * Ci}, x.dt);
+    widen_bias();
     k_pack_w256<<<dim3(Ci / 64, 27, Co / 32), 256, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Ci);
     a.w = wpack.ptr<uint16_t>();
     const SpConvCache::RowTable& rt = c.row_table(-1);
@@ -2424,7 +2441,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     a.tsched = c.tile_schedule(-1, 256).ptr<int32_t>();
   } else if (cfg.BK == 64 && Co % 128 == 0) {  // wide kernels read the 32x32x16-ordered weight copy
     wpack = empty({(i64)Co * 27 * Ci}, x.dt);
-    k_pack_w<<<dim3(Ci / 64 * 2, 27, Co / 64), 256, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci);
+    k_pack_w<<<dim3(Ci / 64 * 2, 27, Co / 64), 256, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Ci, bc);
     a.w = wpack.ptr<uint16_t>();
     // the kernel reads its tiles' neighbour rows from the sorted-order table
     const SpConvCache::RowTable& rt = c.row_table(-1);
@@ -2439,8 +2456,10 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
   // the generic kernel reads the reference's per-block offset masks (valid(B1)'s OR masks); the others do not
   if (!ht && !(Co == 64 && Ci <= 128) && !(Co % 256 == 0 && Ci % 64 == 0 && w256_enabled()) &&
       !(Co % 256 == 0 && Ci % 32 == 0 && w8_enabled()) &&
-      !(cfg.BK == 64 && Co % 128 == 0))
+      !(cfg.BK == 64 && Co % 128 == 0)) {
+    widen_bias();
     a.code = c.block_masks(cfg.B1).ptr<uint32_t>();
+  }
   if (ln) {
     a.ln_on = 1;
     a.ln_gamma = ln->gamma ? ln->gamma->ptr<float>() : nullptr;
