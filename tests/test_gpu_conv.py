@@ -524,6 +524,30 @@ def test_bias_16bit(gpu, ci, co, bias_dt):
     run_case(gpu, shell(9.0), ci, co, in_dt=bias_dt, act=1, bias_dt=bias_dt, seed=ci + co)
 
 
+@pytest.mark.parametrize("ci", [32, 96, 128])
+@pytest.mark.parametrize("n", [1, 255, 257, 5000])
+def test_narrow_first_and_later(gpu, ci, n):
+    """Ci -> 64 of the gathering kernel: a cache's first conv reads the kernel map itself, the second builds the
+    tile-order table and reads that; the same bits, plain and gathered through a row map, and the oracle's result."""
+    c = W.shell_coords(W.CONFIGS["c3"])[:n]
+    nbr, _, _, _ = oracle.build_neighbors(c)
+    cfg = W.Config("t", 0, 0, (0, 0), False, 0, ci, 64, "bf16", "", 90 + ci)
+    w, b = W.conv_params(cfg)
+    tx, qx = quantize(W.features(n, ci, 91), "bf16")
+    tw, qw = quantize(w, "bf16")
+    tb, qb = quantize(b, "f32")
+    tx, tw, tb, tc = (t.to(gpu) for t in (tx, tw, tb, torch.from_numpy(c)))
+    rmap = torch.randperm(n + 3, generator=torch.Generator().manual_seed(n))[:n].int()  # entries past n read zeros
+    qg = np.where((rmap < n).numpy()[:, None], qx[rmap.clamp(max=n - 1).long().numpy()], 0)
+    for gathered in (False, True):
+        cache = sp.build_neighbors(tc)
+        call = ((lambda: sp.subm_conv_gathered(tx, rmap.to(gpu), 0, tw, tb, cache, out_dtype=torch.float32)) if gathered
+                else (lambda: sp.subm_conv_fused(tx, tw, tb, cache, out_dtype=torch.float32)))
+        first = call()
+        assert torch.equal(first, call()) and torch.equal(first, call())
+        compare(first, oracle.conv(qg if gathered else qx, qw, qb, nbr), "f32", f"narrow ci={ci} n={n}")
+
+
 def test_wide_tail_split_256_f16(gpu, monkeypatch):
     """256 -> 256, fp16, bias + SiLU on the first 80000 rows of the C3 shell: 625 single-channel-tile row tiles,
     79 per XCD (72 on the last), so the last 15 (8) tiles of each XCD are split along K over 4 (8) workgroups on a

@@ -545,6 +545,11 @@ __global__ void __launch_bounds__(64) k_pack_w_narrow(const u32x4* __restrict__ 
 //    two offsets ahead with the other savings, still two workgroups per CU: 0.923). Same sums, same bits.
 // Copies rows [row0, row0+BM) of the tile-ordered neighbour table (27 u32 per row, contiguous) into LDS by DMA:
 // 16 bytes per lane, so each wavefront instruction moves 1 KiB with no registers involved.
+// 4 bytes per lane, global -> LDS: lane l's land at dst + l (dst uniform over the wavefront)
+__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t* dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, off, 0, 0, kStreamed);
+}
+
 template <int BM, int NT>
 __device__ __forceinline__ void dma_tile_table(const ConvArgs& a, int row0, uint32_t* srcT, int tid) {
   constexpr int TU = BM * 27 / 4;  // 16-byte units
@@ -613,16 +618,29 @@ __global__ void __launch_bounds__(256, LITE ? 3 : 1) k_conv_narrow(ConvArgs a) {
 
   // prologue: the tile's block of the neighbour table goes to LDS by DMA; rows, 16-row masks from the same order
   // (the table is padded to whole tiles, except nbr itself for spill tiles: rows past N read zeros there, which the
-  // zero mask of those rows keeps out of every result)
-  dma_tile_table<BM, NT>(a, row0, srcT, tid);
+  // zero mask of those rows keeps out of every result). Without a table (a cache's first conv, see conv_impl) the
+  // rows' neighbour indices come straight from nbr, one dependent round trip later.
+  if (a.tbl) dma_tile_table<BM, NT>(a, row0, srcT, tid);
   if (tid < BM) {
     const int row = row0 + tid;
     const bool live = row < N;
-    ordT[tid] = live ? (a.order ? a.order[row] : row) : 0;
-    uint32_t gm = live ? a.gs[row] : 0u;
+    const int o = live ? (a.order ? a.order[row] : row) : 0;
+    ordT[tid] = o;
+    uint32_t gm = live ? (a.tbl ? a.gs[row] : a.gray[o]) : 0u;
 #pragma unroll
     for (int d = 1; d < 16; d <<= 1) gm |= (uint32_t)__shfl_xor((int)gm, d, 64);
     if ((tid & 15) == 0) gmask[tid >> 4] = gm;
+  }
+  if (!a.tbl) {
+    __syncthreads();  // ordT
+    const __amdgpu_buffer_rsrc_t rn = make_rsrc(a.nbr, a.nbr_bytes);
+    constexpr int NE = BM * SR, PER = (NE + NT - 1) / NT;
+#pragma unroll
+    for (int k = 0; k < PER; k++) {
+      const int e = k * NT + tid, r = e / SR;
+      const uint32_t off = r < BM && row0 + r < N ? (uint32_t)ordT[r] * 108u + (uint32_t)(e - r * SR) * 4u : kOutOfRange;
+      if (k * NT + wv * 64 < NE) dma4(rn, &srcT[k * NT + wv * 64], off);
+    }
   }
   wait_vmcnt<0>();  // this lane's table DMA has landed (the barrier below covers the other lanes)
   __syncthreads();
@@ -2407,11 +2425,18 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     k_pack_w_narrow<<<dim3(Ci / 32, Co / 16, 27), 64, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci,
                                                                      bc, a.kcontig);
     a.w = wpack.ptr<uint16_t>();
-    const SpConvCache::RowTable& rt = c.row_table(16);
-    a.order = rt.order.ptr<int32_t>();
-    a.tbl = rt.tbl.ptr<uint32_t>();
-    a.gs = rt.gs.ptr<int32_t>();
-    a.tbl_bytes = (uint32_t)rt.tbl.bytes();
+    // The tile-order table pays from the second conv on a cache on: building it moves 216 bytes per row (1.7 M children
+    // 107 us), reading nbr through the order costs each tile a round trip (children 128 -> 64: kernel 707 -> 769 us, call 1081 -> 1020).
+    if (c.narrow_calls++ == 0 && !c.rtab.count(16)) {
+      a.order = c.window_order(16).ptr<int32_t>();
+      a.tbl = nullptr;
+    } else {
+      const SpConvCache::RowTable& rt = c.row_table(16);
+      a.order = rt.order.ptr<int32_t>();
+      a.tbl = rt.tbl.ptr<uint32_t>();
+      a.gs = rt.gs.ptr<int32_t>();
+      a.tbl_bytes = (uint32_t)rt.tbl.bytes();
+    }
     if (row_map) {  // the kernel maps each tile's neighbour rows in its prologue (no mapped copy of the table)
       a.rmap = row_map->ptr<int32_t>();
       a.rshift = shift;

@@ -40,6 +40,7 @@ struct SpConvCache {
     Tensor order, tbl, gs;
   };
   std::map<int, RowTable> rtab;
+  int narrow_calls = 0;  // convs of the gathering kernel so far: the first one reads nbr itself
   const RowTable& row_table(int log2w);
   // Tiles of B consecutive entries of row_table(log2w) in dispatch order: longest first (by the number of offsets
   // in the tile's union mask, the tile's K stages), so the last workgroups of a launch are the short ones.
