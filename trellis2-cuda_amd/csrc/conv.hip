@@ -1978,13 +1978,14 @@ __global__ void __launch_bounds__(256) k_split_reduce256(ConvArgs a) {
 // 128-row tiles, two workgroups per CU. Measured on C3 (1526 tiles of 256 rows): 256-row tiles with one workgroup
 // per CU were 6% slower (prologue, barriers and epilogue exposed; 2x fewer weight loads per flop did not make up
 // for it), as were 8 wavefronts of 128 rows x 64 channels on a 256-row tile (3% slower: weights loaded twice).
-// Reduction of the split tiles: one thread per (row, 8 channels) of a split tile; sums its pieces' partials in
-// piece order, then the fused epilogue (bias, act, residual, one rounding) of the unsplit kernel.
+// Reduction of the split tiles: one thread per two (row, 8 channels) segments of a split tile; sums their pieces'
+// partials in piece order, then the fused epilogue (bias, act, residual, one rounding) of the unsplit kernel. Bound by
+// the partials' bytes once enough of them are in flight: two segments per thread instead of one took 4 to 5 us off
+// 1024 -> 4096 at 1803 rows (438 -> 433 with its LayerNorm) and a 512-channel block of 11467 rows (238 -> 233).
 template <int BM, int BN>
 __global__ void __launch_bounds__(256) k_split_reduce(ConvArgs a) {
-  constexpr int UPT = BM * BN / 8 / 256;  // workgroups per split tile
-  int st = blockIdx.x / UPT;                 // split tile, counted over the XCDs in order
-  const int e8 = (blockIdx.x % UPT) * 256 + threadIdx.x, r = e8 / (BN / 8), c8 = e8 % (BN / 8) * 8;
+  constexpr int U = 2, UPT = BM * BN / 8 / 256 / U;  // row segments per thread, workgroups per split tile
+  int st = blockIdx.x / UPT;                         // split tile, counted over the XCDs in order
   int x = 0, ntail = 0;
   for (; x < 8; x++) {
     ntail = a.xk[x] > 1 ? (a.xt0[x + 1] - a.xt0[x]) - a.xs : 0;
@@ -1995,26 +1996,39 @@ __global__ void __launch_bounds__(256) k_split_reduce(ConvArgs a) {
   const int kx = a.xk[x], logical = a.xt0[x] + a.xs + st, pbase = a.xpart0[x] + st * kx;
   const int tm_ = a.tnmaj ? logical % a.tiles_m : logical / a.tiles_n;
   const int tn_ = a.tnmaj ? logical / a.tiles_m : logical % a.tiles_n;
-  const int row = tm_ * BM + r, col = tn_ * BN + c8;
-  float v[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-  for (int j = 0; j < kx; j++) {
-    const float* pp = a.part + ((size_t)(pbase + j) * BM + r) * BN + c8;
-    const f32x4 lo = *(const f32x4*)pp, hi = *(const f32x4*)(pp + 4);
-#pragma unroll
-    for (int q = 0; q < 4; q++) {
-      v[q] += lo[q];
-      v[q + 4] += hi[q];
-    }
-  }
-  const bool ok = row < a.N;
   const Epi e = make_epi(a);
+  const int e8 = (blockIdx.x % UPT) * (256 * U) + threadIdx.x;  // segments e8 and e8 + 256: the same columns
+  const int c8 = e8 % (BN / 8) * 8, col = tn_ * BN + c8;
+  static_assert(256 % (BN / 8) == 0, "a thread's segments share their columns");
+  float v[U][8] = {};
+  uint32_t o[U];
+  bool ok[U];
+  u32x4 rv[U][2];
+#pragma unroll
+  for (int u = 0; u < U; u++) {
+    const int row = tm_ * BM + (e8 + u * 256) / (BN / 8);
+    ok[u] = row < a.N;
+    o[u] = (uint32_t)(ok[u] ? a.order[row] : 0) * (uint32_t)a.Co + (uint32_t)col;
+  }
+#pragma unroll 2
+  for (int j = 0; j < kx; j++)
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const float* pp = a.part + ((size_t)(pbase + j) * BM + (e8 + u * 256) / (BN / 8)) * BN + c8;
+      const f32x4 lo = *(const f32x4*)pp, hi = *(const f32x4*)(pp + 4);
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        v[u][q] += lo[q];
+        v[u][q + 4] += hi[q];
+      }
+    }
   float bias8[8];
 #pragma unroll
   for (int q = 0; q < 8; q++) bias8[q] = a.bias ? a.bias[col + q] : 0.f;
-  const uint32_t o = (uint32_t)(ok ? a.order[row] : 0) * (uint32_t)a.Co + (uint32_t)col;
-  u32x4 rv[2];
-  load_res8(e, o, ok, rv);
-  store_row8(e, o, ok, v, bias8, rv);
+#pragma unroll
+  for (int u = 0; u < U; u++) load_res8(e, o[u], ok[u], rv[u]);
+#pragma unroll
+  for (int u = 0; u < U; u++) store_row8(e, o[u], ok[u], v[u], bias8, rv[u]);
 }
 
 int device_cus() {
@@ -2097,7 +2111,7 @@ void launch_wide_dma(ConvArgs a) {
     int ntail = 0;
     for (int x = 0; x < 8; x++)
       if (a.xk[x] > 1) ntail += (a.xt0[x + 1] - a.xt0[x]) - a.xs;
-    k_split_reduce<BM, BN><<<ntail * (BM * BN / 8 / 256), 256, 0, stream()>>>(a);
+    k_split_reduce<BM, BN><<<ntail * (BM * BN / 8 / 512), 256, 0, stream()>>>(a);
   }
 }
 
