@@ -527,8 +527,8 @@ def test_bias_16bit(gpu, ci, co, bias_dt):
 @pytest.mark.parametrize("ci", [32, 96, 128])
 @pytest.mark.parametrize("n", [1, 255, 257, 5000])
 def test_narrow_first_and_later(gpu, ci, n):
-    """Ci -> 64 of the gathering kernel: a cache's first conv reads the kernel map itself, the second builds the
-    tile-order table and reads that; the same bits, plain and gathered through a row map, and the oracle's result."""
+    """Ci -> 64 of the gathering kernel: a cache's first conv reads the kernel map itself and writes the tile-order
+    table, the later ones read that; the same bits, plain and gathered through a row map, and the oracle's result."""
     c = W.shell_coords(W.CONFIGS["c3"])[:n]
     nbr, _, _, _ = oracle.build_neighbors(c)
     cfg = W.Config("t", 0, 0, (0, 0), False, 0, ci, 64, "bf16", "", 90 + ci)
@@ -546,6 +546,30 @@ def test_narrow_first_and_later(gpu, ci, n):
         first = call()
         assert torch.equal(first, call()) and torch.equal(first, call())
         compare(first, oracle.conv(qg if gathered else qx, qw, qb, nbr), "f32", f"narrow ci={ci} n={n}")
+
+
+@pytest.mark.parametrize("first,later", [(128, 32), (32, 128), (96, 96)])
+@pytest.mark.parametrize("n", [1, 100, 128, 129, 300, 511, 5000])
+def test_narrow_table_after_first(gpu, first, later, n):
+    """A cache's first gathering conv leaves its schedules complete: the second allocates what the third does, whatever
+    the tiles of the first (128 rows at Ci = 128, else 256), and convs that read the table through a row map
+    (its padding is EMPTY, never a row number) give the bits of a fresh cache's first conv."""
+    tc = torch.from_numpy(W.shell_coords(W.CONFIGS["c3"])[:n]).to(gpu)
+    g = torch.Generator(device=gpu).manual_seed(n)
+    r = lambda *s: torch.randn(s, generator=g, device=gpu).to(torch.bfloat16)
+    rmap = torch.randperm(n, generator=torch.Generator().manual_seed(n)).int().to(gpu)
+    x1, w1, x2, w2 = r(n, first), r(64, 27, first), r(n, later), r(64, 27, later)
+    cache = sp.build_neighbors(tc)
+    sp.subm_conv(x1, w1, None, cache)
+    call = lambda ca: sp.subm_conv_gathered(x2, rmap, 0, w2, None, ca)
+    at = [sp.alloc_counts()[0]]
+    ys = []
+    for _ in range(3):
+        ys.append(call(cache))
+        at.append(sp.alloc_counts()[0])
+    assert at[1] - at[0] == at[2] - at[1] == at[3] - at[2]
+    fresh = call(sp.build_neighbors(tc))
+    assert all(torch.equal(y, fresh) for y in ys)
 
 
 def test_wide_tail_split_256_f16(gpu, monkeypatch):

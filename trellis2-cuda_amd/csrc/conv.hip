@@ -125,6 +125,9 @@ struct ConvArgs {
   const int32_t* order;
   const uint32_t* tbl;  // neighbour table in tile order (SpConvCache::row_table), for the kernels that use it
   const int32_t* gs;    // neighbour masks in tile order
+  uint32_t* tbl_out;    // without tbl (k_conv_narrow): where the kernel writes the table and the masks it read through
+  int32_t* gs_out;      // the order, padded to npad rows
+  int npad;
   const int32_t* gray;
   const uint32_t* code;
   const int32_t* hrows;    // halo schedule (SpConvCache::halo_table), for k_conv_halo
@@ -619,7 +622,7 @@ __global__ void __launch_bounds__(256, LITE ? 3 : 1) k_conv_narrow(ConvArgs a) {
   // prologue: the tile's block of the neighbour table goes to LDS by DMA; rows, 16-row masks from the same order
   // (the table is padded to whole tiles, except nbr itself for spill tiles: rows past N read zeros there, which the
   // zero mask of those rows keeps out of every result). Without a table (a cache's first conv, see conv_impl) the
-  // rows' neighbour indices come straight from nbr, one dependent round trip later.
+  // rows' neighbour indices come straight from nbr, one dependent round trip later, and leave as the table's block.
   if (a.tbl) dma_tile_table<BM, NT>(a, row0, srcT, tid);
   if (tid < BM) {
     const int row = row0 + tid;
@@ -627,6 +630,7 @@ __global__ void __launch_bounds__(256, LITE ? 3 : 1) k_conv_narrow(ConvArgs a) {
     const int o = live ? (a.order ? a.order[row] : row) : 0;
     ordT[tid] = o;
     uint32_t gm = live ? (a.tbl ? a.gs[row] : a.gray[o]) : 0u;
+    if (!a.tbl) a.gs_out[row] = (int32_t)gm;  // npad is a multiple of the tile's rows
 #pragma unroll
     for (int d = 1; d < 16; d <<= 1) gm |= (uint32_t)__shfl_xor((int)gm, d, 64);
     if ((tid & 15) == 0) gmask[tid >> 4] = gm;
@@ -644,6 +648,23 @@ __global__ void __launch_bounds__(256, LITE ? 3 : 1) k_conv_narrow(ConvArgs a) {
   }
   wait_vmcnt<0>();  // this lane's table DMA has landed (the barrier below covers the other lanes)
   __syncthreads();
+  if (!a.tbl) {
+    if (row0 + BM > N) {  // the last tile: its rows past N are EMPTY, and so is the padding past it
+      for (int e = (N - row0) * SR + tid; e < BM * SR; e += NT) srcT[e] = EMPTY;
+      const i64 pad = (i64)row0 + BM;
+      for (i64 e = pad * SR + tid; e < (i64)a.npad * SR; e += NT) a.tbl_out[e] = EMPTY;
+      for (i64 r = pad + tid; r < a.npad; r += NT) a.gs_out[r] = 0;
+      __syncthreads();
+    }
+    constexpr int TU = BM * SR / 4;  // 16-byte units
+    u32x4* to = (u32x4*)(a.tbl_out + (i64)row0 * SR);
+#pragma unroll
+    for (int k = 0; k < (TU + NT - 1) / NT; k++) {
+      const int u = k * NT + tid;
+      if (u < TU) to[u] = *(const u32x4*)&srcT[u * 4];
+    }
+    if (a.rmap) __syncthreads();  // srcT is rewritten below
+  }
   if (a.rmap) {  // gathered conv: the tile's neighbour rows become source rows row_map[r] >> shift (EMPTY past rmax)
     constexpr int NE = BM * SR, PER = (NE + NT - 1) / NT;
     uint32_t mv[PER];
@@ -2402,6 +2423,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
   a.Co = Co;
   a.act = act;
   Tensor wpack, mtbl;
+  SpConvCache::RowTable fresh;  // a table that this call's kernel writes: the cache's once the kernel is queued
   REQ(!row_map || reads_row_table(cfg, Ci, Co, act), "row map with a kernel that reads nbr directly");
   const SpConvCache::HaloTable* ht = nullptr;
   if (Co == 64 && Ci == 64 && halo_enabled()) ht = &c.halo_table(HaloShape<2>::B, HaloShape<2>::UM);
@@ -2439,13 +2461,20 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     k_pack_w_narrow<<<dim3(Ci / 32, Co / 16, 27), 64, 0, stream()>>>((const u32x4*)w.p, (u32x4*)wpack.p, Co, Ci,
                                                                      bc, a.kcontig);
     a.w = wpack.ptr<uint16_t>();
-    // The tile-order table pays from the second conv on a cache on: building it moves 216 bytes per row (1.7 M children
-    // 107 us), reading nbr through the order costs each tile a round trip (children 128 -> 64: kernel 707 -> 769 us, call 1081 -> 1020).
-    if (c.narrow_calls++ == 0 && !c.rtab.count(16)) {
-      a.order = c.window_order(16).ptr<int32_t>();
-      a.tbl = nullptr;
+    // A cache's first conv reads nbr through the order and writes the tile-order table on the way, so that every later
+    // one finds it. A pass of its own for the table moves 216 bytes per row (1.7 M children 107 us) where this costs
+    // each tile a round trip: subdivision, map and one conv of 1.7 M children 128 -> 64, 1152 us with the pass (and
+    // the slower sort of then) against 1050. Reading nbr and writing nothing was 1030, but the second conv then paid
+    // for the pass: map and two convs of 1.2 M rows 1907 us against 1836, at 96 -> 64 1460 against 1383.
+    const auto it = c.rtab.find(16);
+    if (it == c.rtab.end()) {
+      fresh = c.new_row_table(16);
+      a.order = fresh.order.ptr<int32_t>();
+      a.tbl_out = fresh.tbl.ptr<uint32_t>();
+      a.gs_out = fresh.gs.ptr<int32_t>();
+      a.npad = (int)fresh.gs.numel();
     } else {
-      const SpConvCache::RowTable& rt = c.row_table(16);
+      const SpConvCache::RowTable& rt = it->second;
       a.order = rt.order.ptr<int32_t>();
       a.tbl = rt.tbl.ptr<uint32_t>();
       a.gs = rt.gs.ptr<int32_t>();
@@ -2543,6 +2572,7 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
   else dispatch<false>(cfg, a);
   CK(hipGetLastError());
   ktimer_mark();
+  if (a.tbl_out) c.rtab.emplace(16, fresh);
 }
 
 void subm_conv_skip(const Tensor& x, const Tensor& w, const Tensor* b, int act, const Tensor& x_skip,

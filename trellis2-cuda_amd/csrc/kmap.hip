@@ -695,16 +695,22 @@ __global__ void __launch_bounds__(256) k_row_table(const uint32_t* __restrict__ 
   }
 }
 
+SpConvCache::RowTable SpConvCache::new_row_table(int log2w) {
+  RowTable r;
+  r.order = log2w < 0 ? sorted : window_order(log2w);
+  const i64 npad = std::max<i64>(cdiv(N, kRowTablePad), 1) * kRowTablePad;
+  REQ(npad * 108 <= 0xfffe0000ll, "neighbour table of %lld rows too large", (long long)npad);
+  r.tbl = empty({npad, 27}, I32);
+  r.gs = empty({npad}, I32);
+  return r;
+}
+
 const SpConvCache::RowTable& SpConvCache::row_table(int log2w) {
   const int key = log2w < 0 ? -1 : log2w;
   auto it = rtab.find(key);
   if (it != rtab.end()) return it->second;
-  RowTable r;
-  r.order = key < 0 ? sorted : window_order(key);
-  const i64 npad = std::max<i64>(cdiv(N, kRowTablePad), 1) * kRowTablePad;
-  r.tbl = empty({npad, 27}, I32);
-  r.gs = empty({npad}, I32);
-  REQ(npad * 108 <= 0xfffe0000ll, "neighbour table of %lld rows too large", (long long)npad);
+  RowTable r = new_row_table(key);
+  const i64 npad = r.gs.numel();
   k_row_table<<<cdiv(npad, 36), 256, 0, stream()>>>(nbr.ptr<uint32_t>(), gray.ptr<int32_t>(),
                                                     r.order.ptr<int32_t>(), N, N, npad, r.tbl.ptr<uint32_t>(),
                                                     r.gs.ptr<int32_t>());

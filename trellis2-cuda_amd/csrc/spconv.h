@@ -40,8 +40,8 @@ struct SpConvCache {
     Tensor order, tbl, gs;
   };
   std::map<int, RowTable> rtab;
-  int narrow_calls = 0;  // convs of the gathering kernel so far: the first one reads nbr itself
   const RowTable& row_table(int log2w);
+  RowTable new_row_table(int log2w);  // the same, not filled and not memoized (a kernel that writes it follows)
   // Tiles of B consecutive entries of row_table(log2w) in dispatch order: longest first (by the number of offsets
   // in the tile's union mask, the tile's K stages), so the last workgroups of a launch are the short ones.
   // Memoized per (log2w, B).
