@@ -135,6 +135,16 @@ def test_sort_small(gpu, n):
         assert torch.equal(a, b)
 
 
+@pytest.mark.parametrize("step,edge", [(1, 11), (1, 29), (3, 29), (2, 27)])
+def test_sort_one_digit(gpu, step, edge):
+    """Up to 24576 rows whose masks are mostly one (a solid cube) or all one (voxels apart), rows shuffled: the one-launch
+    sort passes add a wavefront's equal digits together; map, masks and order bit-exact."""
+    r = np.arange(edge, dtype=np.int32) * step
+    p = np.stack(np.meshgrid(r, r, r, indexing="ij"), -1).reshape(-1, 3)
+    c = np.concatenate([np.zeros((len(p), 1), np.int32), p], 1)
+    check_map(np.ascontiguousarray(c[np.random.default_rng(edge).permutation(len(c))]), gpu, B1s=(128,))
+
+
 @pytest.mark.parametrize("name", ["c1", "c5"])
 def test_subdivide(gpu, name):
     par = coords(name)

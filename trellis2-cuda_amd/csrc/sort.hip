@@ -208,11 +208,15 @@ __global__ void __launch_bounds__(DPW* TG) k_rs_digit_scan(const uint32_t* __res
 
 // One pass in one launch, for few keys: every workgroup (1024 keys, one chunk per wavefront) counts the digits of all
 // n keys itself, those of the tiles before its own apart, which gives its tile starts without a count and a scan
-// launch; ranks and destinations are the scatter kernel's.
+// launch; ranks and destinations are the scatter kernel's. The counting bounds it, and in it the lanes of a wavefront
+// that add to one LDS counter: one after the other, up to 64 of them, since solid shapes hold mostly one mask and shells
+// few. So the two digits held by the first lanes are each added once by one of their lanes (kernel map of 24000 rows:
+// shell 58.5 -> 51.9 us, solid cube 84.9 -> 40.8, all children of 3000 parents 89.7 -> 66.5; one such digit 53.0 /
+// 44.9 / 71.6, three 52.4 / 41.1 / 70).
 __global__ void __launch_bounds__(1024) k_rs_pass(const uint32_t* __restrict__ kin, const int32_t* __restrict__ vin,
                                                   uint32_t* __restrict__ kout, int32_t* __restrict__ vout, int n,
                                                   int shift, const uint32_t* __restrict__ ndev) {
-  constexpr int NW = 16;
+  constexpr int NW = 16, U = 4, LEAD = 2;
   __shared__ uint32_t cnt[NW][NBUK], before[NBUK], rest[NBUK], red[NBUK / 64];
   if (ndev) n = min((uint32_t)n, *ndev);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6, base = blockIdx.x * 1024;
@@ -220,8 +224,30 @@ __global__ void __launch_bounds__(1024) k_rs_pass(const uint32_t* __restrict__ k
   for (int d = lane; d < NBUK; d += 64) cnt[wv][d] = 0;
   if (tid < NBUK) before[tid] = rest[tid] = 0;
   __syncthreads();
-#pragma unroll 4
-  for (int i = tid; i < n; i += 1024) atomicAdd(&(i < base ? before : rest)[(kin[i] >> shift) & (NBUK - 1)], 1u);
+  for (int i0 = 0; i0 < n; i0 += 1024 * U) {
+    uint32_t k[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) k[u] = i0 + u * 1024 + tid < n ? kin[i0 + u * 1024 + tid] : 0u;
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int i1 = i0 + u * 1024;
+      if (i1 + tid >= n) break;
+      uint32_t* c = i1 < base ? before : rest;
+      const uint32_t d = (k[u] >> shift) & (NBUK - 1);
+      bool mine = true;  // not added yet
+#pragma unroll
+      for (int l = 0; l < LEAD; l++) {
+        if (!mine) break;
+        const uint32_t first = __builtin_amdgcn_readfirstlane(d);
+        const uint64_t peers = __ballot(d == first);
+        if (d == first) {
+          mine = false;
+          if (lane == __builtin_ctzll(peers)) atomicAdd(&c[d], (uint32_t)__popcll(peers));
+        }
+      }
+      if (mine) atomicAdd(&c[d], 1u);
+    }
+  }
   uint32_t key[1], rank[1];
   int32_t val[1];
   rank_chunks<1>(kin, vin, n, shift, base + wv * 64, lane, cnt[wv], key, val, rank);
@@ -255,8 +281,9 @@ __global__ void __launch_bounds__(1024) k_rs_pass(const uint32_t* __restrict__ k
     vout[pos] = val[0];
   }
 }
-// Kernel map and quads of n voxels, one launch per pass / three: 8000 44 / 62 us, 15000 52 / 63, 20000 58 / 64, 30000
-// 70 / 64, 60000 115 / 66: counting all keys in every workgroup pays up to ~24 k of them.
+// Kernel map of n voxels, one launch per pass / three, us: shell 8000 36 / 57, 16000 44 / 58, 20000 47 / 58, 24000
+// 52 / 57, 28000 55 / 59, 34000 62 / 59; all children kept 16000 60 / 80, 24000 67 / 81, 34000 77 / 83: counting all keys
+// in every workgroup pays up to ~24 k of them.
 constexpr i64 kSmallKeys = 1024 * 24;
 }  // namespace
 
