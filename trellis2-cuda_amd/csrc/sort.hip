@@ -127,7 +127,9 @@ __global__ void __launch_bounds__(RT) k_rs_scatter(const uint32_t* __restrict__ 
 // exclusive tile starts in `start` (not in place: the counts stay intact for such a fallback read).
 // It is bound by its dependent round trips, not by bytes. With digit-major counts and one workgroup per digit, every
 // tile's 512 counts and starts were 512 separate lines, for the count and the scatter kernel too: 1.2 M keys, count
-// 10.3 -> 6.6 us, scan 10.8 -> 9.2, scatter 10.8 -> 9.2.
+// 10.3 -> 6.6 us, scan 10.8 -> 9.2, scatter 10.8 -> 9.2. The held counts' loops end at the run's length, the same for all
+// threads: walked to their full 32, builds of 25 to 60 k rows were 1 to 2 us slower than digit-major (40000 rows, whole
+// build: digit-major 58.7, full walk 59.6, as it is 55.5).
 constexpr int DPW = 16, TG = 64, HELD = 32;  // digits per workgroup, tile groups, counts held by a thread
 __global__ void __launch_bounds__(DPW* TG) k_rs_digit_scan(const uint32_t* __restrict__ cnt,
                                                            uint32_t* __restrict__ start, uint64_t* __restrict__ dsum,
@@ -139,11 +141,15 @@ __global__ void __launch_bounds__(DPW* TG) k_rs_digit_scan(const uint32_t* __res
   const int dd = tid % DPW, g = tid / DPW, per = (ntiles + TG - 1) / TG;
   const int t0 = min(g * per, ntiles), t1 = min(t0 + per, ntiles);
   const uint32_t* col = cnt + d0 + dd;
-  uint32_t mine = 0, c[HELD];  // a short run is read once, all of it in flight, and held; a long one read twice
+  uint32_t mine = 0, c[HELD] = {};  // a short run is read once, all of it in flight, and held; a long one read twice
   const bool held = per <= HELD;
   if (held) {
 #pragma unroll
-    for (int k = 0; k < HELD; k++) c[k] = t0 + k < t1 ? col[(i64)(t0 + k) * NBUK] : 0u;
+    for (int k0 = 0; k0 < HELD; k0 += 4) {
+      if (k0 >= per) break;
+#pragma unroll
+      for (int k = k0; k < k0 + 4; k++) c[k] = t0 + k < t1 ? col[(i64)(t0 + k) * NBUK] : 0u;
+    }
 #pragma unroll
     for (int k = 0; k < HELD; k++) mine += c[k];
   } else {
@@ -192,9 +198,13 @@ __global__ void __launch_bounds__(DPW* TG) k_rs_digit_scan(const uint32_t* __res
   uint32_t* out = start + d0 + dd;
   if (held) {
 #pragma unroll
-    for (int k = 0; k < HELD; k++) {
-      if (t0 + k < t1) out[(i64)(t0 + k) * NBUK] = run;
-      run += c[k];
+    for (int k0 = 0; k0 < HELD; k0 += 4) {
+      if (k0 >= per) break;
+#pragma unroll
+      for (int k = k0; k < k0 + 4; k++) {
+        if (t0 + k < t1) out[(i64)(t0 + k) * NBUK] = run;
+        run += c[k];
+      }
     }
     return;
   }
@@ -281,8 +291,8 @@ __global__ void __launch_bounds__(1024) k_rs_pass(const uint32_t* __restrict__ k
     vout[pos] = val[0];
   }
 }
-// Kernel map of n voxels, one launch per pass / three, us: shell 8000 36 / 57, 16000 44 / 58, 20000 47 / 58, 24000
-// 52 / 57, 28000 55 / 59, 34000 62 / 59; all children kept 16000 60 / 80, 24000 67 / 81, 34000 77 / 83: counting all keys
+// Kernel map of n voxels, one launch per pass / three, us: shell 8000 36 / 53, 16000 44 / 54, 20000 47 / 54, 24000
+// 52 / 53, 28000 56 / 55, 34000 62 / 55; all children kept 16000 60 / 73, 24000 67 / 75, 34000 78 / 77: counting all keys
 // in every workgroup pays up to ~24 k of them.
 constexpr i64 kSmallKeys = 1024 * 24;
 }  // namespace
