@@ -346,6 +346,27 @@ def test_grid_sample_ragged(gpu, L):
         assert bool(((y - xv.sum(1)).abs() <= 8 * 2.0 ** -24 * xv.abs().sum(1) + 1e-30).all()), C
 
 
+@pytest.mark.parametrize("L", [2 ** 28 + 1, 2 ** 29 + 37])
+def test_grid_sample_many(gpu, L):
+    """More points than one launch covers: 8 threads per point pass 2^32 threads at 2^29 points. 2^20 points over and over;
+    every repetition's rows and weights are those of a call with the 2^20 alone."""
+    c = coords("c1")
+    P = 1 << 20
+    g = torch.Generator(device=gpu).manual_seed(7)
+    base = torch.rand((P, 3), generator=g, device=gpu) * 34 - 1
+    pts = torch.empty((L, 3), device=gpu)
+    for a in range(0, L, P):
+        pts[a:a + P] = base[:min(P, L - a)]
+    cache = sp.build_neighbors(torch.from_numpy(c).to(gpu), 32, 32, 32, keep_hash=True)
+    nb0, wt0 = sp.grid_sample_map(cache, base)
+    nb, wt = sp.grid_sample_map(cache, pts)
+    same = torch.ones((), dtype=torch.bool, device=gpu)
+    for a in range(0, L, P):
+        m = min(P, L - a)
+        same &= (nb[a:a + m] == nb0[:m]).all() & (wt[a:a + m] == wt0[:m]).all()
+    assert bool(same) and int((nb0 >= 0).sum()) > P // 8
+
+
 @pytest.mark.parametrize("name", ["c1", "c5"])
 def test_subdivide_build(gpu, name):
     """subdivide_build (no host sync between the subdivision and the map build: launches sized for the 8n-child

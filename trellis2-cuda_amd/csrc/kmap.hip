@@ -574,11 +574,15 @@ void grid_sample_map(const SpConvCache& c, const Tensor& grid, int batch, bool n
   REQ(nb.numel() == L * 8 && wt.dt == F32 && wt.numel() == L * 8, "nb must be u32 [L,8], wt f32 [L,8]");
   if (L == 0) return;
   REQ(c.N == 0 || c.htable.defined(), "the cache was built without keep_hash");
-  k_grid_sample_map<<<cdiv(L, 32), 256, 0, stream()>>>(
-      grid.ptr<float>(), L, batch, c.W, c.H, c.D, c.N ? (const ulonglong2*)c.htable.p : nullptr, c.hmask,
-      c.hmaskd.defined() ? c.hmaskd.ptr<uint32_t>() : nullptr, c.N ? c.hbricks.ptr<uint32_t>() : nullptr, normalize,
-      nb.ptr<uint32_t>(), wt.ptr<float>());
-  CK(hipGetLastError());
+  constexpr i64 kPart = 1ll << 28;  // points per launch: a launch holds fewer than 2^32 threads
+  for (i64 at = 0; at < L; at += kPart) {
+    const i64 m = std::min(kPart, L - at);
+    k_grid_sample_map<<<cdiv(m, 32), 256, 0, stream()>>>(
+        grid.ptr<float>() + at * 3, m, batch, c.W, c.H, c.D, c.N ? (const ulonglong2*)c.htable.p : nullptr, c.hmask,
+        c.hmaskd.defined() ? c.hmaskd.ptr<uint32_t>() : nullptr, c.N ? c.hbricks.ptr<uint32_t>() : nullptr, normalize,
+        nb.ptr<uint32_t>() + at * 8, wt.ptr<float>() + at * 8);
+    CK(hipGetLastError());
+  }
 }
 
 void grid_sample_sum(const Tensor& x, const Tensor& nb, const Tensor& wt, Tensor& y) {
