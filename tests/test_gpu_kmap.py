@@ -320,9 +320,9 @@ def test_fdg_quads_fill(gpu):
     assert torch.equal(quad[has], keep[has]) and bool((quad[~has] == -1).all()) and bool((keep[~has] == 77).all())
 
 
-@pytest.mark.parametrize("L", [1, 31, 32, 33, 63, 65, 4000])
+@pytest.mark.parametrize("L", [1, 31, 32, 33, 63, 65, 127, 129, 4000])
 def test_grid_sample_ragged(gpu, L):
-    """Point counts around the sample map's 64-point workgroup, points that are not finite among them: rows and
+    """Point counts around the sample map's wavefront (32 points) and workgroup (128), points that are not finite among them: rows and
     weights equal those of the same points inside a longer call, nothing is written past L, and the normalized weights
     are the corner-order sum's quotients. Sums for channel counts of every vector width, reading an x at a 4-byte
     offset, are the float32 fused multiply-add chain: within 8 roundings of the float64 sum."""
@@ -344,6 +344,31 @@ def test_grid_sample_ragged(gpu, L):
         y = sp.grid_sample_sum(x, nb, wt).double()
         xv = torch.where((nb >= 0)[:, :, None], x[nb.clamp(min=0).long()], 0.0).double() * wt.double()[:, :, None]
         assert bool(((y - xv.sum(1)).abs() <= 8 * 2.0 ** -24 * xv.abs().sum(1) + 1e-30).all()), C
+
+
+@pytest.mark.parametrize("bounds", [(32, 32, 32), (29, 30, 31), (33, 5, 3)])
+@pytest.mark.parametrize("batch", [0, 1])
+def test_grid_sample_rows(gpu, bounds, batch):
+    """The sample map's rows are lookup's of the 8 corners: points in every position inside a 4^3 brick and past each
+    face of the grid (bounds that are no multiple of 4 or cut the voxels off among them), two batches of voxels."""
+    c = coords("c1")
+    c = c[(c[:, 1] < bounds[0]) & (c[:, 2] < bounds[1]) & (c[:, 3] < bounds[2])]
+    have = {tuple(q) for q in c.tolist()}  # and a block that every grid holds
+    block = [(0, x, y, z) for x in (1, 2) for y in (3, 4) for z in (0, 1) if (0, x, y, z) not in have]
+    c = np.concatenate([c, np.array(block, np.int32).reshape(-1, 4)])
+    c2 = c[::-3].copy()
+    c2[:, 0] = 1
+    c = np.ascontiguousarray(np.concatenate([c, c2]), dtype=np.int32)
+    cache = sp.build_neighbors(torch.from_numpy(c).to(gpu), *bounds, keep_hash=True)
+    rng = np.random.default_rng(batch)
+    pts = torch.from_numpy((rng.uniform(-3.0, np.array(bounds) + 3.0, size=(20000, 3))).astype(np.float32)).to(gpu)
+    nb, wt = sp.grid_sample_map(cache, pts, batch=batch)
+    base = torch.floor(pts - 0.5).int()
+    for v in range(8):
+        q = torch.full((len(pts), 4), batch, dtype=torch.int32, device=gpu)
+        q[:, 1:] = base + torch.tensor([v >> 2, v >> 1 & 1, v & 1], device=gpu, dtype=torch.int32)
+        assert torch.equal(nb[:, v], sp.lookup(cache, q)), v
+    assert bool(((wt != 0) <= (nb >= 0)).all()) and int((nb >= 0).sum()) > 0
 
 
 @pytest.mark.parametrize("L", [2 ** 28 + 1, 2 ** 29 + 37])

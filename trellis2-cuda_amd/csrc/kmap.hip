@@ -476,41 +476,88 @@ __global__ void __launch_bounds__(256) k_fdg_quads(const uint32_t* __restrict__ 
 // voxel i spans [i, i+1) with its centre at i + 0.5) reads the 8 voxels around u = p - 0.5: corner v = dx*4 + dy*2 +
 // dz of base floor(u), weight ((dx ? fx : 1-fx) * (dy ? fy : 1-fy)) * (dz ? fz : 1-fz), f = u - floor(u). Absent or
 // off-grid corners: EMPTY with weight 0; with `normalize` the present weights are divided by their sum.
-// One lane per (point, corner), the 8 corners of a point in 8 consecutive lanes: a lane makes one probe and one record
-// read (two dependent round trips), lanes of one brick share its lines, and rows and weights leave as full lines. One
-// thread per point walked its 8 corners' round trips one after the other and stored with a 32-byte lane stride: 1 M
-// points in random order near a shell of 0.8 M voxels 242 -> 76 us. What is left is the rate of those random line
-// reads (the table and records are outside L2): two or four points per lane, their reads overlapped, measured level.
+// Two lanes per point, one for each dx, so that rows and weights leave as full lines. Corners in one 4^3 brick share its
+// probe (as a rule all four of a lane), and the probes of the bricks it needs are in flight together, then the records.
+// Points in random order are bound by the rate of those line reads (table and records are outside L2), points in
+// spatial order by the instructions. us for 1 M / 4 M points near a shell of 0.8 M voxels, random and in order: as it is
+// 73, 23 / 270, 98; one lane per corner 70, 40 / 255, 175; one per point, its corners one after the other 212, 34 /
+// 800, 117; one per pair of corners 69, 30 / 256, 135; two lanes that probe one brick after the other 74, 27 / 272, 117.
 __global__ void __launch_bounds__(256) k_grid_sample_map(const float* __restrict__ grid, i64 L, int b, int W, int H,
                                                          int D, const ulonglong2* __restrict__ t, uint32_t mask0,
                                                          const uint32_t* __restrict__ maskp,
                                                          const uint32_t* __restrict__ bricks, bool normalize,
                                                          uint32_t* __restrict__ nb, float* __restrict__ wt) {
-  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x, i = e >> 3;
-  if (i >= L) return;  // the 8 lanes of a point together
-  const int v = threadIdx.x & 7, dx = v >> 2, dy = (v >> 1) & 1, dz = v & 1;
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4), aligned(4)));
+  typedef float f32x4 __attribute__((ext_vector_type(4), aligned(4)));
+  const i64 e = (i64)blockIdx.x * blockDim.x + threadIdx.x, i = e >> 1;
+  if (i >= L) return;  // both lanes of a point
+  const int dx = threadIdx.x & 1;
   const float px = grid[i * 3], py = grid[i * 3 + 1], pz = grid[i * 3 + 2];
-  const bool fin = isfinite(px) && isfinite(py) && isfinite(pz) && fabsf(px) < 1e9f && fabsf(py) < 1e9f &&
-                   fabsf(pz) < 1e9f;
+  const bool fin = fabsf(px) < 1e9f && fabsf(py) < 1e9f && fabsf(pz) < 1e9f;  // false for infinities and NaN
   const float ux = px - 0.5f, uy = py - 0.5f, uz = pz - 0.5f;
   const float bx = floorf(ux), by = floorf(uy), bz = floorf(uz);
   const float fx = ux - bx, fy = uy - by, fz = uz - bz;
-  const int x = (fin ? (int)bx : 0) + dx, y = (fin ? (int)by : 0) + dy, z = (fin ? (int)bz : 0) + dz;
-  uint32_t row = EMPTY;
-  if (fin && t && b >= 0 && x >= 0 && y >= 0 && z >= 0 && x < W && y < H && z < D) {
-    const uint32_t id = brick_find(t, brick_key(b, x, y, z, (W + 3) >> 2, (H + 3) >> 2, (D + 3) >> 2),
-                                   maskp ? *maskp : mask0);
-    if (id != EMPTY) row = bricks[(i64)id * 64 + brick_local(x, y, z)];
+  const int x = (fin ? (int)bx : 0) + dx, y0 = fin ? (int)by : 0, z0 = fin ? (int)bz : 0;
+  u32x4 row = {EMPTY, EMPTY, EMPTY, EMPTY};  // corner j = dy * 2 + dz of this lane
+  if (fin && t && b >= 0 && x >= 0 && x < W) {
+    const uint32_t mask = maskp ? *maskp : mask0;
+    const int D4 = (D + 3) >> 2;
+    const uint64_t k0 = brick_key(b, x, y0, z0, (W + 3) >> 2, (H + 3) >> 2, D4);
+    const bool iny[2] = {y0 >= 0 && y0 < H, y0 >= -1 && y0 + 1 < H}, inz[2] = {z0 >= 0 && z0 < D, z0 >= -1 && z0 + 1 < D};
+    // y0 + 1 (z0 + 1) lies in the brick of y0 (z0), or else in the next one, as it does where y0 = -1
+    const bool ny = ((y0 + 1) & 3) == 0, nz = ((z0 + 1) & 3) == 0;
+    const bool sy = iny[0] && !ny, sz = inz[0] && !nz;  // dy = 1 (dz = 1) takes the brick of dy = 0 (dz = 0)
+    uint64_t k[4];
+    uint32_t at[4], id[4];
+    ulonglong2 q[4];
+    bool own[4];
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int dy = j >> 1, dz = j & 1;
+      own[j] = iny[dy] && inz[dz] && !(dy && sy) && !(dz && sz);
+      k[j] = k0 + (uint64_t)(dy && ny ? D4 : 0) + (uint64_t)(dz && nz ? 1 : 0);
+      at[j] = brick_home(k[j], mask);
+      q[j] = ulonglong2{HEMPTY, 0};
+      if (own[j]) q[j] = t[at[j]];
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      id[j] = EMPTY;
+      if (own[j]) {
+        while (q[j].x != k[j] && q[j].x != HEMPTY) {
+          at[j] = (at[j] + 1) & mask;
+          q[j] = t[at[j]];
+        }
+        if (q[j].x == k[j]) id[j] = (uint32_t)q[j].y;
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++) {
+      const int dy = j >> 1, dz = j & 1;
+      if (!own[j] && iny[dy] && inz[dz]) {
+        const int from = (dy && !sy ? 2 : 0) + (dz && !sz ? 1 : 0);
+        id[j] = from == 0 ? id[0] : from == 1 ? id[1] : id[2];
+      }
+    }
+#pragma unroll
+    for (int j = 0; j < 4; j++)
+      if (id[j] != EMPTY) row[j] = bricks[(i64)id[j] * 64 + brick_local(x, y0 + (j >> 1), z0 + (j & 1))];
   }
-  float w = row == EMPTY ? 0.f : ((dx ? fx : 1.f - fx) * (dy ? fy : 1.f - fy)) * (dz ? fz : 1.f - fz);
-  if (normalize) {  // the sum in corner order, which every lane of the point needs
+  const float wx = dx ? fx : 1.f - fx;
+  f32x4 w;
+#pragma unroll
+  for (int j = 0; j < 4; j++)
+    w[j] = row[j] == EMPTY ? 0.f : (wx * (j >> 1 ? fy : 1.f - fy)) * (j & 1 ? fz : 1.f - fz);
+  if (normalize) {  // the sum in corner order, which both lanes need
     float sum = 0.f;
 #pragma unroll
-    for (int j = 0; j < 8; j++) sum += __shfl(w, j, 8);
-    if (sum > 0.f) w = w / sum;
+    for (int l = 0; l < 2; l++)
+#pragma unroll
+      for (int j = 0; j < 4; j++) sum += __shfl(w[j], l, 2);
+    if (sum > 0.f) w = f32x4{w[0] / sum, w[1] / sum, w[2] / sum, w[3] / sum};
   }
-  nb[e] = row;
-  wt[e] = w;
+  *(u32x4*)(nb + e * 4) = row;
+  *(f32x4*)(wt + e * 4) = w;
 }
 
 // y[i, c] = sum over v = 0..7 of x[nb[i, v], c] * wt[i, v], fused multiply-adds in v order (EMPTY reads 0): the
@@ -577,7 +624,7 @@ void grid_sample_map(const SpConvCache& c, const Tensor& grid, int batch, bool n
   constexpr i64 kPart = 1ll << 28;  // points per launch: a launch holds fewer than 2^32 threads
   for (i64 at = 0; at < L; at += kPart) {
     const i64 m = std::min(kPart, L - at);
-    k_grid_sample_map<<<cdiv(m, 32), 256, 0, stream()>>>(
+    k_grid_sample_map<<<cdiv(m, 128), 256, 0, stream()>>>(
         grid.ptr<float>() + at * 3, m, batch, c.W, c.H, c.D, c.N ? (const ulonglong2*)c.htable.p : nullptr, c.hmask,
         c.hmaskd.defined() ? c.hmaskd.ptr<uint32_t>() : nullptr, c.N ? c.hbricks.ptr<uint32_t>() : nullptr, normalize,
         nb.ptr<uint32_t>() + at * 8, wt.ptr<float>() + at * 8);
