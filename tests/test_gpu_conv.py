@@ -572,6 +572,27 @@ def test_narrow_table_after_first(gpu, first, later, n):
     assert all(torch.equal(y, fresh) for y in ys)
 
 
+@pytest.mark.parametrize("co", [128, 384, 64, 256])
+def test_gathered_large_source(gpu, co):
+    """Source rows of more than 2^32 bytes, past a gather's 32-bit offsets. Co an odd multiple of 128: the rows that are
+    read are copied first, the same bits as a conv of the copied rows. The other widths refuse them."""
+    c = W.shell_coords(W.CONFIGS["c3"])[:5000]
+    n, ci, M = len(c), 64, 33_700_000
+    cache = sp.build_neighbors(torch.from_numpy(c).to(gpu))
+    g = torch.Generator(device=gpu).manual_seed(co)
+    r = lambda *s: torch.randn(s, generator=g, device=gpu).to(torch.bfloat16)
+    rows = torch.randperm(M, generator=g, device=gpu)[:n].int()
+    rows[:2] = torch.tensor([M - 1, M // 2], dtype=torch.int32)
+    src, x, w = torch.zeros((M, ci), dtype=torch.bfloat16, device=gpu), r(n, ci), r(co, 27, ci)
+    src[rows.long()] = x
+    call = lambda: sp.subm_conv_gathered(src, rows << 1, 1, w, None, cache)
+    if co % 256 == 128:
+        assert torch.equal(call(), sp.subm_conv(x, w, None, cache))
+    else:
+        with pytest.raises(RuntimeError, match="larger than"):
+            call()
+
+
 def test_wide_tail_split_256_f16(gpu, monkeypatch):
     """256 -> 256, fp16, bias + SiLU on the first 80000 rows of the C3 shell: 625 single-channel-tile row tiles,
     79 per XCD (72 on the last), so the last 15 (8) tiles of each XCD are split along K over 4 (8) workgroups on a

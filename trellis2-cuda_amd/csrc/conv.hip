@@ -2265,8 +2265,8 @@ SpConvCfg spconv_cfg(int N, int Ci, int Co) {
   return SpConvCfg{128, Ci % 64 == 0 ? 64 : 32, 1};
 }
 
-// The kernels that read their tiles' neighbour rows from the tile-order table (narrow, 256-channel wide) can read
-// them through a row map instead; the others get the gathered rows materialized.
+// The kernels that read their tiles' neighbour rows from the tile-order table (narrow, wide) can read them through a
+// row map instead; the others get the gathered rows materialized.
 bool reads_row_table(const SpConvCfg& cfg, int Ci, int Co, int act) {
   (void)act;
   return (Co == 64 && Ci <= 128) || (cfg.BK == 64 && Co % 128 == 0);
@@ -2609,7 +2609,10 @@ void subm_conv_gathered(const Tensor& x_src, const Tensor& row_map, int shift, c
   REQ(shift >= 0 && shift < 31, "shift=%d", shift);
   const int Ci = (int)x_src.size(1), Co = (int)w.size(0);
   REQ(Ci > 0 && Ci % 32 == 0 && Ci <= kMaxCi, "Ci=%d must be a multiple of 32 (at most %d)", Ci, kMaxCi);
-  if (c.N == 0 || reads_row_table(spconv_cfg(c.N, Ci, Co), Ci, Co, act)) {
+  // Source rows past the 32-bit offsets of a gather: Co = 128 odd copies the rows it reads (all of them may still fit);
+  // the other widths refuse them in conv_impl.
+  const bool copy = Co % 256 == 128 && (uint64_t)x_src.size(0) * Ci * 2 > kMaxBufferBytes;
+  if (c.N == 0 || (!copy && reads_row_table(spconv_cfg(c.N, Ci, Co), Ci, Co, act))) {
     conv_impl(x_src, &row_map, shift, w, b, residual, act, c, out);
     return;
   }
