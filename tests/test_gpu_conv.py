@@ -506,11 +506,12 @@ def test_wide_tail_split(gpu, nrows, monkeypatch):
 
 
 @pytest.mark.parametrize("ci,co,nrows,splits", [(64, 128, 1, True), (64, 384, 129, True), (128, 128, 6000, True),
-                                                (64, 128, 60000, False), (64, 128, 110007, True)])
+                                                (64, 128, 60000, False), (64, 128, 80000, False),
+                                                (64, 128, 110007, True)])
 def test_wide_128_splits(gpu, monkeypatch, ci, co, nrows, splits):
     """The 128 x 128 tiles (Co an odd multiple of 128): one row, a ragged second tile, every tile split along K, no
-    split, and a tail split (110007 rows: 108 tiles on an XCD's 96 slots); fp32, bf16 and residual forms, every row
-    against the oracle."""
+    split with the tiles in row order (59 on an XCD's 96 slots) and longest first (79), and a tail split (110007 rows:
+    108); fp32, bf16 and residual forms, every row against the oracle."""
     c = W.shell_coords(W.CONFIGS["c3"])[:nrows]
     differ = split_vs_unsplit(gpu, monkeypatch, c, ci, co, "bf16", 1, "bf16", 71 + nrows, w256=False)
     if torch.cuda.get_device_properties(0).multi_processor_count == 256 and nrows > 1:

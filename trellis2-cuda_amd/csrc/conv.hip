@@ -2067,11 +2067,31 @@ bool split_enabled() {
   return !(e && e[0] && e[0] != '0');
 }
 
-// Wave-quantization tail: with two workgroups per CU, an XCD (32 CUs, its own L2; workgroup ids are dealt to the
-// 8 XCDs round-robin) runs 64 tiles at once. When an XCD's tiles number between 64 and 96 (C2: 594 tiles, 74-75
-// per XCD), the last ones would run as a thin second round; instead each of them is split over k = 64 / tail
-// (at most 8) workgroups along its K stages, so the second round is as wide as the first and k times shorter.
-// Measured on C2: 0.81 ms with 198 row tiles against 0.59 ms with 170 (510 workgroups, one round).
+// Wave-quantization tail: with two workgroups per CU (three at TN = 1), an XCD (32 CUs, its own L2; workgroup ids are
+// dealt to the 8 XCDs round-robin) runs 64 (96) tiles at once. When an XCD's tiles number between one and one and a half
+// times that (C2: 594 tiles, 74-75 per XCD), the last ones would run as a thin second round; instead each of them is
+// split over k = slots / tail (at most 8) workgroups along its K stages, so the second round is as wide as the first
+// and k times shorter. Measured on C2: 0.81 ms with 198 row tiles against 0.59 ms with 170 (510 workgroups, one round).
+// The longest-first order (SpConvCache::tile_schedule, two launches on a cache's first use) is for the other launches:
+// split ones walk XCD-contiguous ranges, and TN = 1 with at most two thirds of its slots taken starts every tile at
+// once (58000 rows, kept map with the order / without, fresh map: 128 -> 128 59 / 59, 124 / 120 us, 512 -> 128 205 / 205,
+// 271 / 266; 75000 rows 66 / 68, 132 / 131 and 231 / 240, 298 / 303). Map and first conv of that kernel's
+// predecessor, which read the kernel map itself: 124 and 266 us; 512 -> 128 at 50000 rows 251 against 256 now.
+struct WidePlan {
+  int slots, per;    // concurrent workgroups and tiles per XCD
+  bool tail, small;  // split the tiles past the first round; split every tile
+  bool ordered;      // longest tiles first
+};
+WidePlan wide_plan(int N, int Co) {
+  const int TN = Co % 256 == 0 ? 2 : 1, tiles = cdiv(N, 128) * (Co / (128 * TN));
+  WidePlan p{(4 - TN) * (device_cus() / 8), cdiv(tiles, 8), false, false, false};
+  if (split_enabled() && p.slots > 0) {
+    p.tail = p.per > p.slots && p.per - p.slots <= p.slots / 2;
+    p.small = 2 * p.per <= p.slots;
+  }
+  p.ordered = !p.tail && !p.small && (TN == 2 || p.per > p.slots * 2 / 3);
+  return p;
+}
 template <bool F16, int TN>
 void launch_wide_dma(ConvArgs a) {
   constexpr int BM = 128, BN = 128 * TN;
@@ -2080,10 +2100,10 @@ void launch_wide_dma(ConvArgs a) {
   const int tiles = a.tiles_m * a.tiles_n;
   a.grid = (tiles + 7) / 8 * 8;
   a.part = nullptr;
-  const int slots = (4 - TN) * (device_cus() / 8);  // concurrent workgroups per XCD
-  const int per = cdiv(tiles, 8);
+  const WidePlan plan = wide_plan(a.N, a.Co);
+  const int slots = plan.slots, per = plan.per;
   Tensor ws;
-  if (split_enabled() && slots > 0 && per > slots && per - slots <= slots / 2) {
+  if (plan.tail) {
     int units = 0, pslots = 0;
     a.xs = slots;
     for (int x = 0; x < 8; x++) {
@@ -2100,7 +2120,7 @@ void launch_wide_dma(ConvArgs a) {
       a.part = ws.ptr<float>();
       a.grid = 8 * units;
     }
-  } else if (split_enabled() && slots > 0 && 2 * per <= slots) {
+  } else if (plan.small) {
     // too few tiles to fill half the slots (small N, e.g. C2's 85 x 3 tiles): every tile is split along its K
     // stages over k = min(8, slots / c) workgroups, so each XCD runs about `slots` pieces at once
     int units = 0, pslots = 0;
@@ -2120,7 +2140,6 @@ void launch_wide_dma(ConvArgs a) {
       a.grid = 8 * units;
     }
   }
-  if (a.part) a.tsched = nullptr;  // the tail split keeps the XCD-contiguous walk
   a.tnmaj = a.part != nullptr;
   // Longest-first tiles are dealt to the XCDs in runs of 16 consecutive ones instead of one by one: within a mask
   // the gray order is the input (Morton) order, so a run's gathers overlap in that XCD's L2. Same bits; C3 kernel
@@ -2517,7 +2536,8 @@ void conv_impl(const Tensor& x, const Tensor* row_map, int shift, const Tensor& 
     a.tbl = row_map ? mtbl.ptr<uint32_t>() : rt.tbl.ptr<uint32_t>();
     a.gs = rt.gs.ptr<int32_t>();
     a.tbl_bytes = (uint32_t)rt.tbl.bytes();
-    a.tsched = c.tile_schedule(-1, 128).ptr<int32_t>();
+    const WidePlan plan = wide_plan(N, Co);
+    if (plan.ordered) a.tsched = c.tile_schedule(-1, 128).ptr<int32_t>();
   }
   REQ(!skip || ht, "the fused skip residual needs the halo kernel");
   REQ(!ln || (ht && ht->host_spills() == 0), "the fused pre-activation needs the halo kernel with no spill tiles");
