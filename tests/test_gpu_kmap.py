@@ -98,8 +98,8 @@ def test_kmap_random_permutation(gpu):
 
 @pytest.mark.parametrize("n", [524288, 524289])
 def test_kmap_sort_paths(gpu, n):
-    """The stable sort switches from the tile look-back form (at most 256 tiles of 2048 keys) to count/scan/scatter
-    passes above it: both sides of the switch, on a permuted prefix of the c4 shell (ties in non-Morton order)."""
+    """The stable sort's count / scan / scatter passes at ragged sizes around 2^19 keys (512 and 513 tiles of 1024, 8 and 9
+    counts per thread of the digit scan), on a permuted prefix of the c4 shell (ties in non-Morton order)."""
     c = coords("c4")[:n].copy()
     c = c[np.random.default_rng(1).permutation(n)]
     print(f"sort path n={n}", flush=True)
@@ -129,6 +129,24 @@ def test_sort_small(gpu, n):
     par = torch.from_numpy(c[:max(n // 8, 1)]).to(gpu)
     lg = torch.from_numpy(W.keep_logits(len(par), 0.4, n).view(np.int16)).to(gpu).view(torch.float16)
     cc, src, cache = sp.subdivide_build(par, lg)
+    oc, osrc = sp.subdivide(par, lg)
+    assert torch.equal(cc, oc) and torch.equal(src, osrc)
+    for a, b in zip(cache.tensors(), sp.build_neighbors(oc).tensors()):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("limit", [None, "0"])
+def test_sort_long_columns(gpu, monkeypatch, limit):
+    """More than 2048 sort tiles, where the digit scan reads its columns twice: a subdivision's tiles are picked for 3 of 8
+    children, and of 600 k parents about 60% are kept here (2.9 M children, 2800 tiles of 1024). Equal to subdivide +
+    build_neighbors, whose tiles (2048 keys) are few enough to be held; also with the lower digits' sums recomputed."""
+    if limit is not None:
+        monkeypatch.setenv("SPCONV_SORT_SPIN_LIMIT", limit)
+    par = torch.from_numpy(coords("c5")[:600000]).to(gpu)
+    lg = torch.from_numpy(W.keep_logits(len(par), 0.6, 3).view(np.int16)).to(gpu).view(torch.float16)
+    cc, src, cache = sp.subdivide_build(par, lg)
+    assert len(cc) > 2048 * 1024
+    monkeypatch.delenv("SPCONV_SORT_SPIN_LIMIT", raising=False)
     oc, osrc = sp.subdivide(par, lg)
     assert torch.equal(cc, oc) and torch.equal(src, osrc)
     for a, b in zip(cache.tensors(), sp.build_neighbors(oc).tensors()):

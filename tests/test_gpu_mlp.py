@@ -92,6 +92,33 @@ def test_convnext_mlp_wide_tiles(gpu, C, N):
     assert bool((out[N:] == 7.0).all())
 
 
+@pytest.mark.parametrize("C,N", [(256, 9001), (256, 33000), (512, 16400), (1024, 8300), (1024, 1300)])
+@pytest.mark.parametrize("dt", [torch.bfloat16, torch.float16])
+def test_convnext_mlp_wide_no_params(gpu, C, N, dt):
+    """The two-GEMM form without gamma, beta and biases, in both types, with its 128 x 256 tiles (K >= 1024 and a tile per
+    CU: both products at C = 1024, N = 8300, the second at 256, 33000 and 512, 16400) and the smaller ones; against
+    torch fp32 on the GPU, bounds as above."""
+    h, x, _, _, w1, _, w2, _ = (a.to(gpu) for a in make(N, C, dt, torch.float32, C + N))
+    y = sp.convnext_mlp(h, x, None, None, w1, None, w2, None, eps=1e-6).float()
+    em, f32 = (reference(h, x, None, None, w1, None, w2, None, 1e-6, d) for d in (dt, None))
+    r_em, mx, r_32 = rel(y, em), float((y - em).abs().max()), rel(y, f32)
+    print(f"C={C} N={N} {dt}: rel-L2 {r_em:.2e} max-abs {mx:.2e} vs emulated, rel-L2 {r_32:.2e} vs fp32", flush=True)
+    assert r_em <= 2e-3 and mx <= 3e-2 and r_32 <= 1e-2
+
+
+@pytest.mark.parametrize("C,N", [(64, 3001), (128, 3001), (256, 98304), (256, 98305), (256, 200001), (512, 49153),
+                                 (1024, 24700), (1024, 50000)])
+@pytest.mark.parametrize("over", ["h", "x"])
+def test_convnext_mlp_in_place(gpu, C, N, over):
+    """y over h and y over x give the bits of a call with its own output, also with the rows in parts (C >= 256:
+    one to three of at most 192 MB of hidden units), where a part's rows are written before the next part's are read."""
+    dev = [a.to(gpu) for a in make(N, C, torch.bfloat16, torch.float32, C)]
+    y = sp.convnext_mlp(*dev, eps=1e-6)
+    out = dev[0 if over == "h" else 1]
+    got = sp.convnext_mlp(*dev, eps=1e-6, out=out)
+    assert got.data_ptr() == out.data_ptr() and torch.equal(got, y)
+
+
 def test_convnext_mlp_errors(gpu):
     h = torch.zeros((10, 96), dtype=torch.bfloat16, device=gpu)
     w1 = torch.zeros((384, 96), dtype=torch.bfloat16, device=gpu)
