@@ -2268,13 +2268,9 @@ void dispatch(const SpConvCfg& cfg, ConvArgs a) {
   if (a.Co % 256 == 0 && a.Ci % 64 == 0 && w256_enabled()) return launch_w256<F16>(a);
   if (cfg.BK == 64 && a.Co % 256 == 0) return launch_wide_dma<F16, 2>(a);
   if (cfg.BK == 64 && a.Co % 128 == 0) return launch_wide_dma<F16, 1>(a);
-  if (a.Co % 128 == 0) {
-    if (cfg.BK == 64) launch<F16, 128, 128, 2, 2, 64>(a);
-    else launch<F16, 128, 128, 2, 2, 32>(a);
-  } else {
-    if (cfg.BK == 64) launch<F16, 128, 64, 4, 1, 64>(a);
-    else launch<F16, 128, 64, 4, 1, 32>(a);
-  }
+  if (a.Co % 128 == 0) launch<F16, 128, 128, 2, 2, 32>(a);
+  else if (cfg.BK == 64) launch<F16, 128, 64, 4, 1, 64>(a);
+  else launch<F16, 128, 64, 4, 1, 32>(a);
 }
 }  // namespace
 
