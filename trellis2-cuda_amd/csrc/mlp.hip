@@ -9,7 +9,7 @@
 // (one 1 KiB fragment per MFMA; a second block of rows per wavefront does not fit in registers), 58321 rows 162 us
 // against 111 (15000: 86 / 39, 390000: 897 / 721).
 //
-// Work split. A workgroup of 4 wavefronts walks row tiles (persistent grid); each wavefront owns R blocks of 32 rows.
+// Work split. A workgroup of 4 wavefronts walks row tiles (persistent grid); each wavefront owns 32 rows.
 // The hidden dimension is processed in chunks of 32:
 //   GEMM1  H^T[32 hid x 32 rows] = W1[chunk rows, :] · Xn^T      (C/16 v_mfma_f32_32x32x16, K = channels)
 //   H^T    += b1, SiLU, rounded to the operand type
@@ -62,6 +62,8 @@ __device__ __forceinline__ uint32_t pack2(float a, float b) {
   else return __builtin_bit_cast(uint32_t, __builtin_convertvector(f32x2{a, b}, bf16x2));
 }
 __device__ __forceinline__ float silu(float v) { return v * __builtin_amdgcn_rcpf(1.0f + __expf(-v)); }
+
+constexpr int kMlpThreads = 256, kMlpRows = kMlpThreads / 64 * 32;  // rows of a workgroup's tile: 32 per wavefront
 
 template <int C>
 struct MlpShape {
@@ -119,11 +121,12 @@ __global__ void __launch_bounds__(256) k_pack_mlp(const uint16_t* __restrict__ w
 }
 
 // params: f32 [gamma C | beta C | b1 4C | b2 C]
-template <bool F16, int C, int R, int NW>
-__global__ void __launch_bounds__(NW * 64, 2) k_convnext_mlp(const uint16_t* h, const uint16_t* x,
-                                                      uint16_t* y, const u32x4* __restrict__ wp,
-                                                      const float* __restrict__ params, float eps, i64 n, i64 tiles,
-                                                      uint32_t h_bytes, uint32_t x_bytes, uint32_t y_bytes) {
+template <bool F16, int C>
+__global__ void __launch_bounds__(kMlpThreads, 2) k_convnext_mlp(const uint16_t* h, const uint16_t* x, uint16_t* y,
+                                                                 const u32x4* __restrict__ wp,
+                                                                 const float* __restrict__ params, float eps, i64 n,
+                                                                 i64 tiles, uint32_t h_bytes, uint32_t x_bytes,
+                                                                 uint32_t y_bytes) {
   using S = MlpShape<C>;
   __shared__ u32x4 lw[S::LDSQ];
   __shared__ float lp[7 * C];
@@ -132,92 +135,80 @@ __global__ void __launch_bounds__(NW * 64, 2) k_convnext_mlp(const uint16_t* h, 
   const float* s_bt = lp + C;
   const float* s_b1 = lp + 2 * C;
   const float* s_b2 = lp + 6 * C;
-  for (int i = tid; i < 7 * C; i += NW * 64) lp[i] = params[i];
+  for (int i = tid; i < 7 * C; i += kMlpThreads) lp[i] = params[i];
   if constexpr (S::RESIDENT)
-    for (int i = tid; i < S::LDSQ; i += NW * 64) lw[i] = wp[i];
+    for (int i = tid; i < S::LDSQ; i += kMlpThreads) lw[i] = wp[i];
   __syncthreads();
   const __amdgpu_buffer_rsrc_t rh = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(h), 0, (int)h_bytes,
                                                                       0x00020000);
   const __amdgpu_buffer_rsrc_t rx = __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(x), 0, (int)x_bytes,
                                                                       0x00020000);
   const __amdgpu_buffer_rsrc_t ry = __builtin_amdgcn_make_buffer_rsrc(y, 0, (int)y_bytes, 0x00020000);
-  constexpr int SQ = (S::CHUNK + NW * 64 - 1) / (NW * 64);  // staged 16-byte units per thread per chunk (streaming mode)
+  constexpr int SQ = (S::CHUNK + kMlpThreads - 1) / kMlpThreads;  // 16-byte units staged per thread and chunk
 
   for (i64 tile = blockIdx.x; tile < tiles; tile += gridDim.x) {
-    const i64 row0 = tile * (NW * R * 32) + (i64)wave * (R * 32);
+    const i64 row = tile * kMlpRows + wave * 32 + r32;
+    const bool ok = row < n;
     asm volatile("" ::: "memory");  // keeps the per-channel LDS parameter reads inside the loop (no 100-VGPR hoist)
     // rows of h (LayerNorm input) as GEMM1 B operands, and x (residual) in the output layout (at C = 128 only in the
     // epilogue: its registers in the loop would spill)
-    u32x4 xn[R][S::KS];
-    u32x2 xr[R][S::YT][4];
-    auto load_x = [&](int rb) __attribute__((always_inline)) {
-      const i64 row = row0 + rb * 32 + r32;
+    u32x4 xn[S::KS];
+    u32x2 xr[S::YT][4];
+    auto load_x = [&]() __attribute__((always_inline)) {
 #pragma unroll
       for (int tt = 0; tt < S::YT; tt++)
 #pragma unroll
         for (int g = 0; g < 4; g++)
-          xr[rb][tt][g] = __builtin_amdgcn_raw_buffer_load_b64(
-              rx, row < n ? (uint32_t)((row * C + tt * 32 + g * 8 + h8 * 4) * 2) : kOOR, 0, 0);
+          xr[tt][g] = __builtin_amdgcn_raw_buffer_load_b64(
+              rx, ok ? (uint32_t)((row * C + tt * 32 + g * 8 + h8 * 4) * 2) : kOOR, 0, 0);
     };
 #pragma unroll
-    for (int rb = 0; rb < R; rb++) {
-      const i64 row = row0 + rb * 32 + r32;
-      const bool ok = row < n;
-#pragma unroll
-      for (int t = 0; t < S::KS; t++)
-        xn[rb][t] = __builtin_amdgcn_raw_buffer_load_b128(rh, ok ? (uint32_t)((row * C + t * 16 + h8 * 8) * 2) : kOOR,
-                                                          0, 0);
-      if constexpr (C == 64) load_x(rb);
-    }
+    for (int t = 0; t < S::KS; t++)
+      xn[t] = __builtin_amdgcn_raw_buffer_load_b128(rh, ok ? (uint32_t)((row * C + t * 16 + h8 * 8) * 2) : kOOR, 0,
+                                                    0);
+    if constexpr (C == 64) load_x();
     // LayerNorm: a row's C values sit in lanes r32 and r32 + 32; mean first, then the centred variance
+    float s = 0.f;
 #pragma unroll
-    for (int rb = 0; rb < R; rb++) {
-      float s = 0.f;
+    for (int t = 0; t < S::KS; t++)
 #pragma unroll
-      for (int t = 0; t < S::KS; t++)
+      for (int j = 0; j < 4; j++) s += lo<F16>(xn[t][j]) + hi<F16>(xn[t][j]);
+    s += __shfl_xor(s, 32, 64);
+    const float mean = s * (1.0f / C);
+    float q = 0.f;
 #pragma unroll
-        for (int j = 0; j < 4; j++) s += lo<F16>(xn[rb][t][j]) + hi<F16>(xn[rb][t][j]);
-      s += __shfl_xor(s, 32, 64);
-      const float mean = s * (1.0f / C);
-      float q = 0.f;
+    for (int t = 0; t < S::KS; t++)
 #pragma unroll
-      for (int t = 0; t < S::KS; t++)
+      for (int j = 0; j < 4; j++) {
+        const float a = lo<F16>(xn[t][j]) - mean, b = hi<F16>(xn[t][j]) - mean;
+        q += a * a + b * b;
+      }
+    q += __shfl_xor(q, 32, 64);
+    const float rstd = rsqrtf(q * (1.0f / C) + eps);
 #pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const float a = lo<F16>(xn[rb][t][j]) - mean, b = hi<F16>(xn[rb][t][j]) - mean;
-          q += a * a + b * b;
-        }
-      q += __shfl_xor(q, 32, 64);
-      const float rstd = rsqrtf(q * (1.0f / C) + eps);
+    for (int t = 0; t < S::KS; t++)
 #pragma unroll
-      for (int t = 0; t < S::KS; t++)
-#pragma unroll
-        for (int j = 0; j < 4; j++) {
-          const int ch = t * 16 + h8 * 8 + 2 * j;
-          const float a = (lo<F16>(xn[rb][t][j]) - mean) * rstd * s_g[ch] + s_bt[ch];
-          const float b = (hi<F16>(xn[rb][t][j]) - mean) * rstd * s_g[ch + 1] + s_bt[ch + 1];
-          xn[rb][t][j] = pack2<F16>(a, b);
-        }
-    }
+      for (int j = 0; j < 4; j++) {
+        const int ch = t * 16 + h8 * 8 + 2 * j;
+        const float a = (lo<F16>(xn[t][j]) - mean) * rstd * s_g[ch] + s_bt[ch];
+        const float b = (hi<F16>(xn[t][j]) - mean) * rstd * s_g[ch + 1] + s_bt[ch + 1];
+        xn[t][j] = pack2<F16>(a, b);
+      }
 
-    f32x16 acc[R][S::YT];
+    f32x16 acc[S::YT];
 #pragma unroll
-    for (int rb = 0; rb < R; rb++)
-#pragma unroll
-      for (int tt = 0; tt < S::YT; tt++) acc[rb][tt] = f32x16{};
+    for (int tt = 0; tt < S::YT; tt++) acc[tt] = f32x16{};
 
     // Software pipeline over hidden chunks: GEMM1 of chunk c+1 is issued before the SiLU of chunk c, so the VALU
     // work overlaps MFMA execution. Streaming mode keeps three chunk buffers: in iteration c the wavefronts read
     // W1 of chunk c+1 and W2 of chunk c, and chunk c+2 is written into the buffer of chunk c-1.
     auto buf = [&](int c) -> const u32x4* { return S::RESIDENT ? lw + c * S::CHUNK : lw + (c % 3) * S::CHUNK; };
-    auto gemm1 = [&](const u32x4* cw, f32x16 (&hacc)[R]) {
-#pragma unroll
-      for (int rb = 0; rb < R; rb++) hacc[rb] = f32x16{};
+    auto gemm1 = [&](const u32x4* cw, f32x16& hacc) {
+      hacc = f32x16{};
 #pragma unroll
       for (int t = 0; t < S::KS; t++) {
         const u32x4 a = cw[t * 64 + lane];
-#pragma unroll
-        for (int rb = 0; rb < R; rb++) hacc[rb] = mfma32<F16>(a, xn[rb][t], hacc[rb]);
+        hacc = mfma32<F16>(a, xn[t], hacc);
       }
     };
     u32x4 stg[SQ];
@@ -225,11 +216,11 @@ __global__ void __launch_bounds__(NW * 64, 2) k_convnext_mlp(const uint16_t* h, 
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < 2 * SQ; k++)
-        if ((k % SQ) * NW * 64 + tid < S::CHUNK)
-          lw[(k / SQ) * S::CHUNK + (k % SQ) * NW * 64 + tid] = wp[(k / SQ) * S::CHUNK + (k % SQ) * NW * 64 + tid];
+        if ((k % SQ) * kMlpThreads + tid < S::CHUNK)
+          lw[(k / SQ) * S::CHUNK + (k % SQ) * kMlpThreads + tid] = wp[(k / SQ) * S::CHUNK + (k % SQ) * kMlpThreads + tid];
       __syncthreads();
     }
-    f32x16 hnext[R];
+    f32x16 hnext;
     gemm1(buf(0), hnext);
 #pragma unroll 1
     for (int c = 0; c < S::NCH; c++) {
@@ -237,30 +228,25 @@ __global__ void __launch_bounds__(NW * 64, 2) k_convnext_mlp(const uint16_t* h, 
         if (c + 2 < S::NCH)
 #pragma unroll
           for (int k = 0; k < SQ; k++)
-            if (k * NW * 64 + tid < S::CHUNK) stg[k] = wp[(c + 2) * S::CHUNK + k * NW * 64 + tid];
-      f32x16 hacc[R];
-#pragma unroll
-      for (int rb = 0; rb < R; rb++) hacc[rb] = hnext[rb];
+            if (k * kMlpThreads + tid < S::CHUNK) stg[k] = wp[(c + 2) * S::CHUNK + k * kMlpThreads + tid];
+      const f32x16 hacc = hnext;
       if (c + 1 < S::NCH) gemm1(buf(c + 1), hnext);
-      u32x4 hb[R][2];
+      u32x4 hb[2];
 #pragma unroll
-      for (int rb = 0; rb < R; rb++)
+      for (int u = 0; u < 2; u++)
 #pragma unroll
-        for (int u = 0; u < 2; u++)
-#pragma unroll
-          for (int j = 0; j < 4; j++) {
-            const int i = u * 8 + 2 * j;  // accumulators i, i+1: hidden rows (i/4)*8 + h8*4 + i%4 (+1)
-            const int hid = c * 32 + (i >> 2) * 8 + h8 * 4 + (i & 3);
-            hb[rb][u][j] = pack2<F16>(silu(hacc[rb][i] + s_b1[hid]), silu(hacc[rb][i + 1] + s_b1[hid + 1]));
-          }
+        for (int j = 0; j < 4; j++) {
+          const int i = u * 8 + 2 * j;  // accumulators i, i+1: hidden rows (i/4)*8 + h8*4 + i%4 (+1)
+          const int hid = c * 32 + (i >> 2) * 8 + h8 * 4 + (i & 3);
+          hb[u][j] = pack2<F16>(silu(hacc[i] + s_b1[hid]), silu(hacc[i + 1] + s_b1[hid + 1]));
+        }
       const u32x4* cw = buf(c);
 #pragma unroll
       for (int tt = 0; tt < S::YT; tt++)
 #pragma unroll
         for (int u = 0; u < 2; u++) {
           const u32x4 a = cw[S::W1Q + (tt * 2 + u) * 64 + lane];
-#pragma unroll
-          for (int rb = 0; rb < R; rb++) acc[rb][tt] = mfma32<F16>(a, hb[rb][u], acc[rb][tt]);
+          acc[tt] = mfma32<F16>(a, hb[u], acc[tt]);
         }
       // buffer (c+2) % 3 held chunk c-1, last read in iteration c-1, which every wavefront finished before the
       // barrier that ended it; one barrier per chunk publishes the new contents
@@ -268,32 +254,25 @@ __global__ void __launch_bounds__(NW * 64, 2) k_convnext_mlp(const uint16_t* h, 
         if (c + 2 < S::NCH) {
 #pragma unroll
           for (int k = 0; k < SQ; k++)
-            if (k * NW * 64 + tid < S::CHUNK) lw[((c + 2) % 3) * S::CHUNK + k * NW * 64 + tid] = stg[k];
+            if (k * kMlpThreads + tid < S::CHUNK) lw[((c + 2) % 3) * S::CHUNK + k * kMlpThreads + tid] = stg[k];
           __syncthreads();
         }
     }
     // y = x + acc + b2, 4 consecutive channels per (tile, group) as one 8-byte store; rows past n are dropped
-    if constexpr (C != 64)
+    if constexpr (C != 64) load_x();
 #pragma unroll
-      for (int rb = 0; rb < R; rb++) load_x(rb);
+    for (int tt = 0; tt < S::YT; tt++)
 #pragma unroll
-    for (int rb = 0; rb < R; rb++) {
-      const i64 row = row0 + rb * 32 + r32;
-      const bool ok = row < n;
-#pragma unroll
-      for (int tt = 0; tt < S::YT; tt++)
-#pragma unroll
-        for (int g = 0; g < 4; g++) {
-          const int co = tt * 32 + g * 8 + h8 * 4;
-          const u32x2 xv = xr[rb][tt][g];
-          const float v0 = acc[rb][tt][g * 4 + 0] + s_b2[co + 0] + lo<F16>(xv[0]);
-          const float v1 = acc[rb][tt][g * 4 + 1] + s_b2[co + 1] + hi<F16>(xv[0]);
-          const float v2 = acc[rb][tt][g * 4 + 2] + s_b2[co + 2] + lo<F16>(xv[1]);
-          const float v3 = acc[rb][tt][g * 4 + 3] + s_b2[co + 3] + hi<F16>(xv[1]);
-          __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2<F16>(v0, v1), pack2<F16>(v2, v3)}, ry,
-                                                ok ? (uint32_t)((row * C + co) * 2) : kOOR, 0, 0);
-        }
-    }
+      for (int g = 0; g < 4; g++) {
+        const int co = tt * 32 + g * 8 + h8 * 4;
+        const u32x2 xv = xr[tt][g];
+        const float v0 = acc[tt][g * 4 + 0] + s_b2[co + 0] + lo<F16>(xv[0]);
+        const float v1 = acc[tt][g * 4 + 1] + s_b2[co + 1] + hi<F16>(xv[0]);
+        const float v2 = acc[tt][g * 4 + 2] + s_b2[co + 2] + lo<F16>(xv[1]);
+        const float v3 = acc[tt][g * 4 + 3] + s_b2[co + 3] + hi<F16>(xv[1]);
+        __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack2<F16>(v0, v1), pack2<F16>(v2, v3)}, ry,
+                                              ok ? (uint32_t)((row * C + co) * 2) : kOOR, 0, 0);
+      }
   }
 }
 
@@ -307,7 +286,7 @@ int device_cus() {
   return n;
 }
 
-template <bool F16, int C, int R, int NW>
+template <bool F16, int C>
 void launch_mlp(const Tensor& h, const Tensor& x, const Tensor& w1, const Tensor& w2, const MlpParams& mp, float eps,
                 Tensor& y) {
   using S = MlpShape<C>;
@@ -315,9 +294,9 @@ void launch_mlp(const Tensor& h, const Tensor& x, const Tensor& w1, const Tensor
   Tensor wp = empty({(i64)S::NCH * S::CHUNK * 8}, h.dt), params = empty({7 * (i64)C}, F32);
   k_pack_mlp<C><<<cdiv(S::NCH * S::CHUNK + 7 * C, 256), 256, 0, stream()>>>(
       w1.ptr<uint16_t>(), w2.ptr<uint16_t>(), mp, (u32x4*)wp.p, params.ptr<float>());
-  const i64 tiles = cdiv(n, (i64)NW * R * 32);
+  const i64 tiles = cdiv(n, kMlpRows);
   const i64 grid = std::min<i64>(tiles, (i64)device_cus() * 2);
-  k_convnext_mlp<F16, C, R, NW><<<(unsigned)grid, NW * 64, 0, stream()>>>(
+  k_convnext_mlp<F16, C><<<(unsigned)grid, kMlpThreads, 0, stream()>>>(
       h.ptr<uint16_t>(), x.ptr<uint16_t>(), y.ptr<uint16_t>(), (const u32x4*)wp.p, params.ptr<float>(), eps, n, tiles,
       (uint32_t)h.bytes(), (uint32_t)x.bytes(), (uint32_t)y.bytes());
 }
@@ -752,7 +731,7 @@ void convnext_mlp(const Tensor& h, const Tensor& x, const Tensor* gamma, const T
   // One 32-row block per wavefront and two wavefronts per SIMD: the SiLU (two quarter-rate operations per hidden unit) of
   // one runs beside the other's MFMAs. Two blocks per wavefront halve C = 128's weight reads from LDS, but take all
   // 512 registers and leave one wavefront per SIMD: 391007 rows 269 us against 197, 60000 rows 51 against 38.
-  if (C == 64) f16 ? launch_mlp<true, 64, 1, 4>(h, x, w1, w2, mp, eps, y) : launch_mlp<false, 64, 1, 4>(h, x, w1, w2, mp, eps, y);
-  else f16 ? launch_mlp<true, 128, 1, 4>(h, x, w1, w2, mp, eps, y) : launch_mlp<false, 128, 1, 4>(h, x, w1, w2, mp, eps, y);
+  if (C == 64) f16 ? launch_mlp<true, 64>(h, x, w1, w2, mp, eps, y) : launch_mlp<false, 64>(h, x, w1, w2, mp, eps, y);
+  else f16 ? launch_mlp<true, 128>(h, x, w1, w2, mp, eps, y) : launch_mlp<false, 128>(h, x, w1, w2, mp, eps, y);
   CK(hipGetLastError());
 }
