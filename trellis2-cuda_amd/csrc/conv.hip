@@ -548,11 +548,6 @@ __global__ void __launch_bounds__(64) k_pack_w_narrow(const u32x4* __restrict__ 
 //    two offsets ahead with the other savings, still two workgroups per CU: 0.923). Same sums, same bits.
 // Copies rows [row0, row0+BM) of the tile-ordered neighbour table (27 u32 per row, contiguous) into LDS by DMA:
 // 16 bytes per lane, so each wavefront instruction moves 1 KiB with no registers involved.
-// 4 bytes per lane, global -> LDS: lane l's land at dst + l (dst uniform over the wavefront)
-__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t* dst, uint32_t off) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, off, 0, 0, kStreamed);
-}
-
 template <int BM, int NT>
 __device__ __forceinline__ void dma_tile_table(const ConvArgs& a, int row0, uint32_t* srcT, int tid) {
   constexpr int TU = BM * 27 / 4;  // 16-byte units
@@ -565,6 +560,10 @@ __device__ __forceinline__ void dma_tile_table(const ConvArgs& a, int row0, uint
       __builtin_amdgcn_raw_ptr_buffer_load_lds(rt, (__attribute__((address_space(3))) void*)&srcT[(k * NT + (tid & ~63)) * 4],
                                                16, base + (uint32_t)u * 16u, 0, 0, kStreamed);
   }
+}
+// 4 bytes per lane, global -> LDS: lane l's land at dst + l (dst uniform over the wavefront)
+__device__ __forceinline__ void dma4(__amdgpu_buffer_rsrc_t r, uint32_t* dst, uint32_t off) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (__attribute__((address_space(3))) void*)dst, 4, off, 0, 0, kStreamed);
 }
 // Byte offset of neighbour row n in a feature matrix with `rowbytes` bytes per row; EMPTY -> past the buffer end
 __device__ __forceinline__ uint32_t nbr_offset(uint32_t n, uint32_t rowbytes) {
