@@ -1335,7 +1335,9 @@ __global__ void __launch_bounds__(256, 4 - TN) k_conv_wide_dma(ConvArgs a) {
   // K stages run channel block outer, offset inner: stage s = (kc = s / nvv, offset entry vi = s % nvv). A row chunk
   // gathered for one offset is then gathered again for the next offset's (one voxel over) neighbours one stage
   // later instead of nkc stages later, while it is still in L2: C3 0.837 -> 0.826 ms, C2 0.297 -> 0.293 (two
-  // interleaved runs; each output's fp32 sum runs over (kc, v) in that order).
+  // interleaved runs; each output's fp32 sum runs over (kc, v) in that order). TN = 1 the other way round / as it is:
+  // 391007 rows of 128 -> 128 311 / 303 us, of 256 -> 128 592 / 557, 110001 rows of 512 -> 128 311 / 287; the error
+  // against 64 bits is the same (bf16 outputs 1.7e-3, fp16 blocks of 128 channels 3.2e-4), the roundings are not.
   int avi = s0 % nvv, akc = s0 / nvv, bvi = avi, bkc = akc, cvi = avi, ckc = akc;
   auto next = [&](int& vi, int& kc) __attribute__((always_inline)) {
     const bool wrap = vi + 1 == nvv;
@@ -2000,8 +2002,9 @@ __global__ void __launch_bounds__(256) k_split_reduce256(ConvArgs a) {
 // for it), as were 8 wavefronts of 128 rows x 64 channels on a 256-row tile (3% slower: weights loaded twice).
 // Reduction of the split tiles: one thread per two (row, 8 channels) segments of a split tile; sums their pieces'
 // partials in piece order, then the fused epilogue (bias, act, residual, one rounding) of the unsplit kernel. Bound by
-// the partials' bytes once enough of them are in flight: two segments per thread instead of one took 4 to 5 us off
-// 1024 -> 4096 at 1803 rows (438 -> 433 with its LayerNorm) and a 512-channel block of 11467 rows (238 -> 233).
+// the partials' bytes once enough of them are in flight: one segment per thread / two, both in turn (runs of one side
+// differ by 0.1 to 0.2%): 1024 -> 4096 at 1803 rows with its LayerNorm 435.2 / 431.2 us, a 512-channel block of 11467
+// rows 238.8 / 234.7, a 1024-channel block of 1803 rows 191.0 / 189.8.
 template <int BM, int BN>
 __global__ void __launch_bounds__(256) k_split_reduce(ConvArgs a) {
   constexpr int U = 2, UPT = BM * BN / 8 / 256 / U;  // row segments per thread, workgroups per split tile
