@@ -2078,7 +2078,9 @@ bool split_enabled() {
 // split ones walk XCD-contiguous ranges, and TN = 1 with at most two thirds of its slots taken starts every tile at
 // once (58000 rows, kept map with the order / without, fresh map: 128 -> 128 59 / 59, 124 / 120 us, 512 -> 128 205 / 205,
 // 271 / 266; 75000 rows 66 / 68, 132 / 131 and 231 / 240, 298 / 303). Map and first conv of that kernel's
-// predecessor, which read the kernel map itself: 124 and 266 us; 512 -> 128 at 50000 rows 251 against 256 now.
+// predecessor, which read the kernel map itself: 124 and 266 us; 512 -> 128 at 50000 rows 251 against 256 now. The one
+// use that a decoder makes of it on a fresh map, an upsample block's second half at 128 channels: 2001 / 6003 / 15001 /
+// 36001 parents 144 / 150 / 165 / 277 us with the predecessor, 98 / 131 / 162 / 259 now.
 struct WidePlan {
   int slots, per;    // concurrent workgroups and tiles per XCD
   bool tail, small;  // split the tiles past the first round; split every tile
